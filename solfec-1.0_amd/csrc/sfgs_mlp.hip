@@ -72,7 +72,8 @@ struct GemmArgs {
   const float *Z; int ldz;              // pre-activations for EPI_GELU_BWD
   int epi;
   int kslice;            // split-K: workgroup z takes K range [z kslice, (z+1) kslice) and writes
-                         // its partial C at C + z M ldc (EPI_F32 only); 0 = whole K
+  size_t zstride;        // its partial C at C + z zstride (EPI_F32 only); 0 = whole K
+  float *colsum;         // when set (split-K): the column sums of B over the K range, at colsum + z zstride
 };
 
 // eight consecutive bf16 of one operand row (16-byte aligned when ld and the
@@ -134,6 +135,11 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs g)
   const int kb = g.kslice ? blockIdx.z*g.kslice : 0, ke = g.kslice ? min(g.K, kb + g.kslice) : g.K;
   floatx4 acc[2][2];
   for (int i = 0; i < 2; i ++) for (int j = 0; j < 2; j ++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  // the first row of workgroups also sums B's columns from the staged tiles (a bias
+  // gradient: one wavefront walking the batch alone took 603 us for 4096 rows, 84 of
+  // the 84.6 ms of 32 minibatches): four threads a column, 8 of the 32 k each
+  const bool sums = g.colsum && blockIdx.y == 0;
+  float cs = 0.f;
 
   for (int k0 = kb; k0 < ke; k0 += BK)
   {
@@ -149,7 +155,20 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs g)
     for (int i = 0; i < 2; i ++)
       for (int j = 0; j < 2; j ++)
         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+    if (sums)
+    {
+      const bf16x8 c = *reinterpret_cast<const bf16x8*>(&Bt[tid >> 2][8*(tid & 3)]);
+      cs += (((float)c[0] + (float)c[1]) + ((float)c[2] + (float)c[3])) +
+            (((float)c[4] + (float)c[5]) + ((float)c[6] + (float)c[7]));
+    }
     __syncthreads();
+  }
+  if (sums)
+  {
+    cs += __shfl_xor(cs, 1, 64);
+    cs += __shfl_xor(cs, 2, 64);
+    const int n = n0 + (tid >> 2);
+    if ((tid & 3) == 0 && n < g.N) g.colsum[(size_t)blockIdx.z*g.zstride + n] = cs;
   }
 
   // epilogue: lane holds D[4(l/16)+q][l%16] of each 16x16 tile
@@ -162,7 +181,7 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs g)
         float v = acc[i][j][q];
         switch (g.epi)
         {
-        case EPI_F32: g.C[((size_t)blockIdx.z*g.M + m)*g.ldc + n] = v; break;
+        case EPI_F32: g.C[(size_t)blockIdx.z*g.zstride + (size_t)m*g.ldc + n] = v; break;
         case EPI_BIAS_F32: g.C[(size_t)m*g.ldc + n] = v + g.bias[n]; break;
         case EPI_BIAS_GELU:
         {
@@ -197,11 +216,13 @@ struct Model {
   int cap = 0;
   bf16 *X = nullptr, *H1 = nullptr, *H2 = nullptr, *H3 = nullptr, *dO = nullptr, *dZ = nullptr, *dZ2 = nullptr;
   float *Z1 = nullptr, *Z2 = nullptr, *Z3 = nullptr, *O = nullptr, *Y = nullptr, *loss = nullptr;
-  float *part = nullptr;   // split-K partials of the weight gradients: ceil(cap / KSLICE) x 128 x 128
+  float *part = nullptr;   // split-K partials of the gradient: up to wgrad_slices(cap) x total
   // device-resident training set
   float *tX = nullptr, *tY = nullptr;
   long long tn = 0, tcap = 0;
   int *idx = nullptr;
+  float *eloss = nullptr;   // the loss partials of one epoch's minibatches
+  size_t eloss_cap = 0;
 };
 
 static void layout(Model &m)
@@ -214,14 +235,19 @@ static void layout(Model &m)
   m.total = o;
 }
 
-// out[i] = sum over the S split-K partials part[z n + i], in z order (deterministic)
+// sum over the S split-K partials part[z n + i], in z order (deterministic)
+__device__ __forceinline__ float sum_parts(int S, size_t n, const float *part, size_t i)
+{
+  float v = 0.0f;
+#pragma unroll 8
+  for (int z = 0; z < S; z ++) v += part[(size_t)z*n + i];
+  return v;
+}
+
 __global__ void k_sum_parts(int S, int n, const float *part, float *out)
 {
   int i = blockIdx.x*blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  float v = 0.0f;
-  for (int z = 0; z < S; z ++) v += part[(size_t)z*n + i];
-  out[i] = v;
+  if (i < n) out[i] = sum_parts(S, n, part, i);
 }
 
 __global__ void k_to_bf16(size_t n, const float *src, bf16 *dst)
@@ -260,25 +286,19 @@ __global__ void k_loss(int B, const float *O, const float *Y, bf16 *dO, float *l
   if (threadIdx.x == 0) loss_part[blockIdx.x] = red[0];
 }
 
-// bias gradient: column sums of a bf16 B x N matrix
-__global__ void k_colsum(int B, int N, const bf16 *D, float *g)
-{
-  int n = blockIdx.x*blockDim.x + threadIdx.x;
-  if (n >= N) return;
-  float s = 0.f;
-  for (int i = 0; i < B; i ++) s += (float)D[(size_t)i*N + n];
-  g[n] = s;
-}
-
-__global__ void k_adam(size_t n, float *p, const float *g, float *m1, float *m2, float lr, float b1, float b2,
-                       float c1, float c2, float eps)
+// one Adam step from the split-K partials of the gradient, with the new bf16
+// copy of the parameters: the gradient itself is not written
+__global__ void k_adam(size_t n, float *p, bf16 *wbf, int S, const float *part, float *m1, float *m2, float lr, float b1,
+                       float b2, float c1, float c2, float eps)
 {
   size_t i = (size_t)blockIdx.x*blockDim.x + threadIdx.x;
   if (i >= n) return;
-  float gi = g[i];
+  float gi = sum_parts(S, n, part, i);
   float a = b1*m1[i] + (1.f - b1)*gi, v = b2*m2[i] + (1.f - b2)*gi*gi;
   m1[i] = a; m2[i] = v;
-  p[i] -= lr * (a/c1) / (sqrtf(v/c2) + eps);
+  const float w = p[i] - lr * (a/c1) / (sqrtf(v/c2) + eps);
+  p[i] = w;
+  wbf[i] = (bf16)w;
 }
 
 // minibatch gather from the resident training set: normalised features -> bf16 X (B x 32), targets Y
@@ -468,13 +488,20 @@ void sfgs_mlp_release(sfgs_ctx *ctx)
   Model *m = (Model*)ctx->mlp;
   if (!m) return;
   void *ptrs[] = {m->param, m->grad, m->m1, m->m2, m->wbf, m->dnorm, m->part, m->X, m->H1, m->H2, m->H3, m->dO, m->dZ, m->dZ2,
-                  m->Z1, m->Z2, m->Z3, m->O, m->Y, m->loss, m->tX, m->tY, m->idx};
+                  m->Z1, m->Z2, m->Z3, m->O, m->Y, m->loss, m->tX, m->tY, m->idx, m->eloss};
   for (void *p : ptrs) if (p) (void)hipFree(p);
   delete m;
   ctx->mlp = nullptr;
 }
 
-static const int KSLICE = 512;   // K per workgroup of a split-K weight-gradient product
+// A weight gradient contracts over the batch, with an output of at most 128 x
+// 128 (four tiles): the batch is split over workgroups in slices of 128 rows, a
+// multiple of the tile's K, so that a batch of 4096 fills 128 of them (8 slices of
+// 512 left 32 workgroups with 16 dependent tile steps each: 13.0 us a product on
+// average over the pass, 8.8 with 128).  Large batches take longer slices, at most
+// 64 of them, which bounds the partials.
+static int wgrad_slice(int B) { return std::max(128, ((B + 63)/64 + BK - 1)/BK*BK); }
+static int wgrad_slices(int B) { return (B + wgrad_slice(B) - 1)/wgrad_slice(B); }
 
 static int gemm(sfgs_ctx *ctx, const GemmArgs &g)
 {
@@ -483,19 +510,16 @@ static int gemm(sfgs_ctx *ctx, const GemmArgs &g)
   return 0;
 }
 
-// a weight gradient C = A' B (small M x N, K = the batch): K split over
-// workgroups in slices of KSLICE, the partials summed in slice order into out
-static int gemm_wgrad(sfgs_ctx *ctx, Model *m, GemmArgs g, float *out)
+// a weight gradient C = A' B of layer l (0..3) and its bias gradient (the column
+// sums of B) into the split-K partials, at their places in the parameter vector
+static int gemm_wgrad(sfgs_ctx *ctx, Model *m, GemmArgs g, int l)
 {
-  const int S = (g.K + KSLICE - 1)/KSLICE;
   g.ldc = g.N;
-  if (S <= 1) { g.C = out; return gemm(ctx, g); }
-  g.kslice = KSLICE;
-  g.C = m->part;
-  gemm(ctx, g);
-  const int n = g.M*g.N;
-  hipLaunchKernelGGL(k_sum_parts, dim3((n + 255)/256), dim3(256), 0, ctx->stream, S, n, m->part, out);
-  return 0;
+  g.kslice = wgrad_slice(g.K);
+  g.zstride = m->total;
+  g.C = m->part + m->off[2*l];
+  g.colsum = m->part + m->off[2*l + 1];
+  return gemm(ctx, g);
 }
 
 static GemmArgs gargs(int M, int N, int K, const bf16 *A, int lda, int tA, const bf16 *B, int ldb, int tB, int epi)
@@ -525,7 +549,8 @@ static int ensure_batch(sfgs_ctx *ctx, Model *m, int B)
   }
   if (m->part) (void)hipFree(m->part);
   m->part = nullptr;
-  HIPCHK(hipMalloc(&m->part, sizeof(float)*(size_t)NH*NH*(size_t)((cap + KSLICE - 1)/KSLICE)));
+  // a smaller batch can take more, shorter slices than the capacity: 64 at most
+  HIPCHK(hipMalloc(&m->part, sizeof(float)*m->total*64));
   m->cap = cap;
   return 0;
 }
@@ -550,36 +575,32 @@ static int forward(sfgs_ctx *ctx, Model *m, int B)
   return 0;
 }
 
-// backward pass from m->dO (bf16) into m->grad (FP32); forward activations must be current
+// backward pass from m->dO (bf16) into the wgrad_slices(B) partials of the
+// gradient in m->part; forward activations must be current
 static int backward(sfgs_ctx *ctx, Model *m, int B)
 {
   const bf16 *W2 = m->wbf + m->off[2], *W3 = m->wbf + m->off[4], *W4 = m->wbf + m->off[6];
-  float *G = m->grad;
   // layer 4
   GemmArgs g = gargs(NH, NOP, B, m->H3, NH, 1, m->dO, NOP, 0, EPI_F32);     // dW4 = H3' dO
-  gemm_wgrad(ctx, m, g, G + m->off[6]);
-  hipLaunchKernelGGL(k_colsum, dim3(1), dim3(64), 0, ctx->stream, B, NOP, m->dO, G + m->off[7]);
+  gemm_wgrad(ctx, m, g, 3);
   g = gargs(B, NH, NOP, m->dO, NOP, 0, W4, NOP, 1, EPI_GELU_BWD);          // dZ3 = (dO W4') * gelu'(Z3)
   g.H = m->dZ; g.ldh = NH; g.Z = m->Z3; g.ldz = NH;
   gemm(ctx, g);
   // layer 3
   g = gargs(NH, NH, B, m->H2, NH, 1, m->dZ, NH, 0, EPI_F32);               // dW3 = H2' dZ3
-  gemm_wgrad(ctx, m, g, G + m->off[4]);
-  hipLaunchKernelGGL(k_colsum, dim3(2), dim3(64), 0, ctx->stream, B, NH, m->dZ, G + m->off[5]);
+  gemm_wgrad(ctx, m, g, 2);
   g = gargs(B, NH, NH, m->dZ, NH, 0, W3, NH, 1, EPI_GELU_BWD);             // dZ2 = (dZ3 W3') * gelu'(Z2)
   g.H = m->dZ2; g.ldh = NH; g.Z = m->Z2; g.ldz = NH;
   gemm(ctx, g);
   // layer 2
   g = gargs(NH, NH, B, m->H1, NH, 1, m->dZ2, NH, 0, EPI_F32);              // dW2 = H1' dZ2
-  gemm_wgrad(ctx, m, g, G + m->off[2]);
-  hipLaunchKernelGGL(k_colsum, dim3(2), dim3(64), 0, ctx->stream, B, NH, m->dZ2, G + m->off[3]);
+  gemm_wgrad(ctx, m, g, 1);
   g = gargs(B, NH, NH, m->dZ2, NH, 0, W2, NH, 1, EPI_GELU_BWD);            // dZ1 = (dZ2 W2') * gelu'(Z1)
   g.H = m->dZ; g.ldh = NH; g.Z = m->Z1; g.ldz = NH;
   gemm(ctx, g);
   // layer 1
   g = gargs(NI, NH, B, m->X, NI, 1, m->dZ, NH, 0, EPI_F32);                // dW1 = X' dZ1
-  gemm_wgrad(ctx, m, g, G + m->off[0]);
-  hipLaunchKernelGGL(k_colsum, dim3(2), dim3(64), 0, ctx->stream, B, NH, m->dZ, G + m->off[1]);
+  gemm_wgrad(ctx, m, g, 0);
   return 0;
 }
 
@@ -716,6 +737,8 @@ int SFGS_Mlp_Grad(sfgs_ctx *ctx, const float *features, const float *targets, in
   int lb = (n + 255)/256;
   hipLaunchKernelGGL(k_loss, dim3(lb), dim3(256), 0, ctx->stream, n, m->O, m->Y, m->dO, m->loss);
   backward(ctx, m, n);
+  hipLaunchKernelGGL(k_sum_parts, dim3((unsigned)((m->total + 255)/256)), dim3(256), 0, ctx->stream, wgrad_slices(n),
+                     (int)m->total, m->part, m->grad);
   std::vector<float> lp((size_t)lb);
   HIPCHK(hipMemcpyAsync(lp.data(), m->loss, sizeof(float)*(size_t)lb, hipMemcpyDeviceToHost, ctx->stream));
   if (grad) HIPCHK(hipMemcpyAsync(grad, m->grad, sizeof(float)*m->total, hipMemcpyDeviceToHost, ctx->stream));
@@ -759,8 +782,17 @@ int SFGS_Mlp_Train(sfgs_ctx *ctx, const float *features, const float *targets, l
   HIPCHK(hipMemcpyAsync(m->tY, targets, sizeof(float)*NO*(size_t)n, hipMemcpyHostToDevice, st));
   std::vector<int> perm((size_t)n);
   unsigned long long s = seed;
-  const int lbmax = (batch + 255)/256;
-  std::vector<float> lp((size_t)lbmax);
+  const int lbmax = (batch + 255)/256, S = wgrad_slices(batch);
+  // the epoch's loss partials stay on the device until its end: no wait per minibatch
+  const size_t nloss = (size_t)(n/batch)*(size_t)lbmax;
+  if (nloss > m->eloss_cap)
+  {
+    if (m->eloss) (void)hipFree(m->eloss);
+    m->eloss = nullptr; m->eloss_cap = 0;
+    HIPCHK(hipMalloc(&m->eloss, sizeof(float)*nloss));
+    m->eloss_cap = nloss;
+  }
+  std::vector<float> lp(nloss);
   const float b1 = 0.9f, b2 = 0.999f;
   for (int e = 0; e < epochs; e ++)
   {
@@ -776,23 +808,23 @@ int SFGS_Mlp_Train(sfgs_ctx *ctx, const float *features, const float *targets, l
     HIPCHK(hipMemcpyAsync(m->idx, perm.data(), sizeof(int)*(size_t)n, hipMemcpyHostToDevice, st));
     double esum = 0.0;
     long long cnt = 0;
-    for (long long b0 = 0; b0 + batch <= n; b0 += batch)
+    float *loss = m->eloss;
+    for (long long b0 = 0; b0 + batch <= n; b0 += batch, loss += lbmax)
     {
       hipLaunchKernelGGL(k_gather, dim3((batch + 255)/256), dim3(256), 0, st, batch, m->idx + b0, m->tX, m->tY, dn,
                          m->X, m->Y);
       forward(ctx, m, batch);
-      hipLaunchKernelGGL(k_loss, dim3(lbmax), dim3(256), 0, st, batch, m->O, m->Y, m->dO, m->loss);
+      hipLaunchKernelGGL(k_loss, dim3(lbmax), dim3(256), 0, st, batch, m->O, m->Y, m->dO, loss);
       backward(ctx, m, batch);
       m->step ++;
       float c1 = 1.f - powf(b1, (float)m->step), c2 = 1.f - powf(b2, (float)m->step);
-      hipLaunchKernelGGL(k_adam, dim3((unsigned)((m->total + 255)/256)), dim3(256), 0, st, m->total, m->param, m->grad,
-                         m->m1, m->m2, lr, b1, b2, c1, c2, 1e-8f);
-      refresh_bf16(ctx, m);
-      HIPCHK(hipMemcpyAsync(lp.data(), m->loss, sizeof(float)*(size_t)lbmax, hipMemcpyDeviceToHost, st));
-      HIPCHK(hipStreamSynchronize(st));
-      for (float v : lp) esum += v;
+      hipLaunchKernelGGL(k_adam, dim3((unsigned)((m->total + 255)/256)), dim3(256), 0, st, m->total, m->param, m->wbf, S,
+                         m->part, m->m1, m->m2, lr, b1, b2, c1, c2, 1e-8f);
       cnt += (long long)batch*NO;
     }
+    HIPCHK(hipMemcpyAsync(lp.data(), m->eloss, sizeof(float)*nloss, hipMemcpyDeviceToHost, st));
+    HIPCHK(hipStreamSynchronize(st));
+    for (float v : lp) esum += v;
     if (loss_hist) loss_hist[e] = cnt ? (float)(esum / (double)cnt) : 0.f;
   }
   HIPCHK(hipGetLastError());
