@@ -102,6 +102,8 @@ __device__ __forceinline__ bool grid_wait(unsigned *bar, unsigned target, int *a
 template <typename T, int G>
 __global__ __launch_bounds__(BAR_NW*64) void k_bar(BarArgs<T> b)
 {
+  __shared__ T lds_all[BAR_NW][Gather<T>::LDS2];
+  T *lds = lds_all[threadIdx.x >> 6];
   __shared__ double red[3][BAR_NW];
   __shared__ int flag, sweepno, sdone;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -131,10 +133,10 @@ __global__ __launch_bounds__(BAR_NW*64) void k_bar(BarArgs<T> b)
       {
         if (mer)
           sweep_slice<T, G, true, true>(a, s, true, lo, hi, back, &sweepno, a.failkey, a.failcount, &b.ctrl->aborted,
-                                        eu, el, up);
+                                        eu, el, up, lds);
         else
           sweep_slice<T, G, false, true>(a, s, true, lo, hi, back, &sweepno, a.failkey, a.failcount,
-                                         &b.ctrl->aborted, eu, el, up);
+                                         &b.ctrl->aborted, eu, el, up, lds);
       }
       if (ci == b.ncol - 1)
       {

@@ -134,7 +134,7 @@ __device__ __forceinline__ int slice_row(const int *row0, const int *nrows, int 
 template <typename T, int G, int NW, bool MERIT>
 __device__ __forceinline__ bool batch_sweep(const BatchGeom &geo, const SweepArgs<T> &a, const BatchScene &sc, int g0,
                                             int w, int nw, int back, int *sweepno, BatchOut *o, unsigned *bar,
-                                            int *flag, double &eu, double &el, double &up)
+                                            int *flag, double &eu, double &el, double &up, T *lds)
 {
   const int wave = threadIdx.x >> 6;
   for (int ci = 0; ci < geo.ncol; ci ++)
@@ -144,7 +144,8 @@ __device__ __forceinline__ bool batch_sweep(const BatchGeom &geo, const SweepArg
     if (s0 == s1) continue;   // same decision in every workgroup of the scene
     const int lo = back ? geo.gptr[gi + 1] : sc.row0, hi = back ? sc.row1 : geo.gptr[gi];
     for (int s = s0 + w*NW + wave; s < s1; s += nw*NW)
-      sweep_slice<T, G, MERIT>(a, s, true, lo, hi, back, sweepno, &o->failkey, &o->failcount, &o->aborted, eu, el, up);
+      sweep_slice<T, G, MERIT>(a, s, true, lo, hi, back, sweepno, &o->failkey, &o->failcount, &o->aborted, eu, el, up,
+                               lds);
     if (!scene_barrier(bar, nw, geo.abort_all, geo.spin_limit, flag)) return false;
   }
   return true;
@@ -159,6 +160,8 @@ __global__ void k_batch_to_f32(long long n, const double *src, float *dst)
 template <typename T, int G, int NW>
 __global__ __launch_bounds__(NW*64) void k_batch(BatchArgs<T> b)
 {
+  __shared__ T lds_all[NW][Gather<T>::LDS2];
+  T *lds = lds_all[threadIdx.x >> 6];
   __shared__ double red[3][NW];
   __shared__ double tot[3];
   __shared__ int flag, sweepno;
@@ -230,9 +233,9 @@ __global__ __launch_bounds__(NW*64) void k_batch(BatchArgs<T> b)
     const int back = b.reverse && (k & 1);
     double eu = 0.0, el = 0.0, up = 0.0;
     if (!b.nomerit && k > 0)
-      alive = batch_sweep<T, G, NW, true>(b.geo, a, sc, g0, w, nw, back, &sweepno, o, bar, &flag, eu, el, up);
+      alive = batch_sweep<T, G, NW, true>(b.geo, a, sc, g0, w, nw, back, &sweepno, o, bar, &flag, eu, el, up, lds);
     else
-      alive = batch_sweep<T, G, NW, false>(b.geo, a, sc, g0, w, nw, back, &sweepno, o, bar, &flag, eu, el, up);
+      alive = batch_sweep<T, G, NW, false>(b.geo, a, sc, g0, w, nw, back, &sweepno, o, bar, &flag, eu, el, up, lds);
     if (!alive) break;
     nsw ++;
     alive = scene_sum(eu, el, up);
@@ -352,10 +355,11 @@ __global__ __launch_bounds__(TPB) void k_usweep(SweepArgs<T> a, const int *clist
   BatchOut *o = out + sc;
   if (o->done) return;                            // a finished scene: whole wavefront
   const int2 bd = sbound[s];
+  __shared__ T lds[TPB/SLICE][MERIT ? Gather<T>::LDS2 : Gather<T>::LDS1];
   double eu = 0.0, el = 0.0, up = 0.0;
   int sweepno = o->iters0 + o->sweeps;
   sweep_slice<T, G, MERIT>(a, s, true, bd.x, bd.y, backward, &sweepno, &o->failkey, &o->failcount, &o->aborted,
-                           eu, el, up);
+                           eu, el, up, lds[threadIdx.x >> 6]);
   eu = wave_sum(eu); el = wave_sum(el); up = wave_sum(up);
   if ((threadIdx.x & 63) == 0)
   {
@@ -494,8 +498,9 @@ template <int G>
 __global__ __launch_bounds__(TPB) void k_umerit(MeritArgs a, int nslices, const int *sscene, const BatchOut *out)
 {
   const int s = blockIdx.x*(TPB/SLICE) + (threadIdx.x >> 6);
+  __shared__ double lds[TPB/SLICE][Gather<double>::LDS1];
   double up = 0.0;
-  merit_slice<G>(a, s, s < nslices && out[sscene[s < nslices ? s : 0]].final_U == 1, up);
+  merit_slice<G>(a, s, s < nslices && out[sscene[s < nslices ? s : 0]].final_U == 1, up, lds[threadIdx.x >> 6]);
 }
 
 struct Tuned { SFGS_BATCH_TUNE t; int valid; };

@@ -75,14 +75,14 @@ struct sfgs_ctx {
   std::vector<int> h_colptr, h_cslice;   // rows / slices per colour (host)
   sfgs::DBuf<unsigned char> scratch;     // hipcub temporary storage
 
-  // ---- slices (SELL-64, colour-major)
+  // ---- slices (64/G rows of one colour each, colour-major)
   int nslices = 0;
-  sfgs::DBuf<int> slice_row0, slice_nrows, slice_len;
+  sfgs::DBuf<int> slice_row0, slice_nrows, slice_len;   // slice_len: blocks of the slice
   sfgs::DBuf<long long> slice_off;       // block offset of slice (in blocks, multiple of 64)
-  long long sell_blocks = 0;             // total block slots incl. padding
+  long long sell_blocks = 0;             // total block slots, the last slot of each slice filled up
 
   // ---- permuted row data (colour-major order)
-  sfgs::DBuf<int> rowlen;                // per permuted row
+  sfgs::DBuf<int> rowlen, rowoff;        // per permuted row: its blocks, the first one's place in the slice
   sfgs::DBuf<double> W, Wd, A, B, V, rho, pfri, pcoh, shift, R, U, Rb, Um;
   int G = 2;                             // lanes per row of the sweep layout (1, 2, 4, 8)
   int wpb = 0;                           // wavefronts per workgroup of the per-colour sweep launches (1, 2, 4;

@@ -146,6 +146,7 @@ template <typename T, int G>
 __global__ __launch_bounds__(64) void k_flow(FlowArgs<T> f)
 {
   const int W = blockIdx.x, lane = threadIdx.x, r = lane / G, g = lane % G;
+  __shared__ T lds[Gather<T>::LDS2];
   const SweepArgs<T> &a0 = f.a;
   for (int k = 0; k < f.maxsweeps; k ++)
   {
@@ -173,15 +174,13 @@ __global__ __launch_bounds__(64) void k_flow(FlowArgs<T> f)
     double eu = 0.0, el = 0.0, up = 0.0;
     for (int s = W; s < f.nslices; s += f.nwaves)
     {
-      // wait for this lane's neighbours: all their versions loaded at once, again
-      // after a pause while any is behind
-      const int row0 = a.row0[s];
+      // wait for the neighbours of this lane's blocks: all their versions loaded at
+      // once, again after a pause while any is behind
+      const int row0 = a.row0[s], total = a.slen[s];
       const bool act = r < a.nrows[s];
       int ok = 1;
-      if (act)
       {
-        const int p = row0 + r, len = a.rowlen[p];
-        const int mine = len > g ? (len - g + G - 1) / G : 0;
+        const int mine = total > lane ? (total - lane + SLICE - 1) / SLICE : 0;
         const int *cb = a.wcol + a.off[s] + lane;
         unsigned spins = 0;
         for (int m0 = 0; m0 < mine && ok; )
@@ -194,7 +193,7 @@ __global__ __launch_bounds__(64) void k_flow(FlowArgs<T> f)
 #pragma unroll
           for (int q = 0; q < CH; q ++) vv[q] = ld_relaxed(f.ver + jj[q]);   // all in flight together
 #pragma unroll
-          for (int q = 0; q < CH; q ++) ready = ready && (m0 + q >= mine || vv[q] >= k + (jj[q] < p ? 1 : 0));
+          for (int q = 0; q < CH; q ++) ready = ready && (m0 + q >= mine || vv[q] >= k + (jj[q] < row0 ? 1 : 0));
           if (ready) { m0 += CH; continue; }
           if (++spins > f.spin_limit) { atomicExch(f.abort_all, 1); ok = 0; break; }
           // a stopped solve leaves rows of later sweeps undone: stop waiting for them
@@ -207,10 +206,10 @@ __global__ __launch_bounds__(64) void k_flow(FlowArgs<T> f)
       // lower-colour neighbours (j < row0 <= p) are read from Q, the rest from P
       if (merit)
         sweep_slice<T, G, true, true>(a, s, true, 0, row0, 0, f.sweepno, a.failkey, a.failcount, &f.ctrl->aborted,
-                                      eu, el, up);
+                                      eu, el, up, lds);
       else
         sweep_slice<T, G, false, true>(a, s, true, 0, row0, 0, f.sweepno, a.failkey, a.failcount, &f.ctrl->aborted,
-                                       eu, el, up);
+                                       eu, el, up, lds);
       publish_fence();
       if (act && g == 0) cst(f.ver + row0 + r, k + 1);
     }

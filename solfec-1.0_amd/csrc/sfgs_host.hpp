@@ -58,7 +58,7 @@ static SweepArgs<T> sweep_args(sfgs_ctx *ctx, const SFGS_PARAM *par, const T *W,
 {
   SweepArgs<T> a;
   a.row0 = ctx->slice_row0.p; a.nrows = ctx->slice_nrows.p; a.rowlen = ctx->rowlen.p; a.off = ctx->slice_off.p;
-  a.slen = ctx->slice_len.p;
+  a.rowoff = ctx->rowoff.p; a.slen = ctx->slice_len.p;
   a.W = W; a.wcol = ctx->wcol.p; a.Wd = Wd; a.A = ctx->A.p; a.B = B; a.rho = rho;
   a.rec = sizeof(T) == 4 ? reinterpret_cast<const float4 *>(ctx->rec32.p) : nullptr;
   a.fri = fri; a.coh = coh; a.shift = shift; a.sep = ctx->sep.p;
@@ -73,6 +73,7 @@ static SweepArgs<T> sweep_args(sfgs_ctx *ctx, const SFGS_PARAM *par, const T *W,
 {
   MeritArgs m;
   m.row0 = ctx->slice_row0.p; m.nrows = ctx->slice_nrows.p; m.rowlen = ctx->rowlen.p; m.off = ctx->slice_off.p;
+  m.rowoff = ctx->rowoff.p; m.slen = ctx->slice_len.p;
   m.W = ctx->W.p; m.wcol = ctx->wcol.p; m.Wd = ctx->Wd.p; m.A = ctx->A.p; m.B = ctx->B.p; m.fri = ctx->pfri.p;
   m.coh = ctx->pcoh.p; m.shift = ctx->shift.p; m.R = ctx->R.p; m.U = ctx->U.p; m.n = ctx->nc; m.update_U = update_U;
   m.mpartials = ctx->mpartials.p; m.conmerit = conmerit;

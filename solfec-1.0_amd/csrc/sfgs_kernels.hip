@@ -6,11 +6,11 @@
 //  * colour-major order (row p = iperm[i]): rows sorted by (colour, -row length,
 //    i); per-row scalars in SoA planes (Wd[e*n + p], B[k*n + p], U[k*n + p]),
 //    reactions R as 4 doubles per row (32-byte aligned gathers);
-//  * off-diagonal blocks in SELL-64: a slice is 64 consecutive rows of one
-//    colour (one wavefront, one row per lane); slot k of lane l stores element e
-//    of its 3x3 block at W[9*off + (9k + e)*64 + l] and the neighbour's row at
-//    wcol[off + 64k + l], so each load instruction of a wave reads 512
-//    contiguous bytes.
+//  * off-diagonal blocks in slices: a slice is 64/G consecutive rows of one
+//    colour (one wavefront, G lanes per row), its blocks row after row without
+//    gaps; block q = 64 m + l of the slice stores element e at
+//    W[9*off + (9m + e)*64 + l] and the neighbour's row at wcol[off + q], so each
+//    load instruction of a wave reads 512 contiguous bytes.
 // One kernel launch sweeps one colour: rows of a colour are not coupled, so the
 // launch order of colours reproduces a serial Gauss-Seidel sweep over the
 // colour-major row order exactly.
@@ -387,20 +387,21 @@ __global__ void k_colour_count(int n, const int *colour, int *count, int ncolour
   for (int c = threadIdx.x; c < ncolours; c += blockDim.x) if (h[c]) atomicAdd(&count[c], h[c]);
 }
 
-__global__ void k_slice_len(int ns, const int *row0, const int *nrows, const int *perm, const int *rowptr, int G,
-                            int *slen, long long *slen_ll)
+// per slice (one wavefront): the place of each row's first block in the slice,
+// the slice's blocks and its block slots (blocks filled up to whole slots)
+__global__ __launch_bounds__(TPB) void k_slice_len(int ns, const int *row0, const int *nrows, const int *perm,
+                                                    const int *rowptr, int *rowoff, int *slen, long long *slen_ll)
 {
-  int s = blockIdx.x*blockDim.x + threadIdx.x;
+  const int s = blockIdx.x*(TPB/SLICE) + (threadIdx.x >> 6), l = threadIdx.x & 63;
   if (s >= ns) return;
-  int len = 0;   // longest row of the slice
-  for (int r = 0; r < nrows[s]; r ++)
-  {
-    int i = perm[row0[s] + r];
-    len = max(len, rowptr[i + 1] - rowptr[i]);
-  }
-  int nslot = (len + G - 1) / G;   // slots of one block per lane
-  slen[s] = nslot;
-  slen_ll[s] = (long long)nslot * SLICE;
+  const int nr = nrows[s], p = row0[s] + l;
+  int len = 0;
+  if (l < nr) { const int i = perm[p]; len = rowptr[i + 1] - rowptr[i]; }
+  int sum = len;   // inclusive prefix sum over the lanes
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) { const int v = __shfl_up(sum, o, 64); if (l >= o) sum += v; }
+  if (l < nr) rowoff[p] = sum - len;
+  if (l == 63) { slen[s] = sum; slen_ll[s] = (long long)((sum + SLICE - 1) / SLICE) * SLICE; }
 }
 
 // =====================================================================
@@ -500,31 +501,53 @@ __global__ __launch_bounds__(TPB) void k_rows(BodyView bv, ConView cv, RowsOut o
 }
 
 struct SellOut {
-  const int *row0, *nrows;
+  const int *row0, *nrows, *rowoff, *slen;
   const long long *off;
   double *W;
   int *wcol;
 };
 
-// off-diagonal blocks W_ij = h s_i s_j H_i^b iM_b H_j^b' (ldy.c:738-844).  G
-// lanes serve one row: lane g of row r (lane l = rG + g) holds blocks k = mG + g
-// in slot m, element e at W[9 off + (9m + e) 64 + l].  The block of a pair is
-// formed with the lower contact index as the "upper" side and transposed for
-// the other, as the reference's symmetry copy (ldy.c:830-844).
-template <int G>
+// the row (0 .. nr - 1) of a slice that holds block q, from the lanes' row
+// offsets (lane r < nr that of row r): the last one that starts at or before q.
+// All lanes of the wavefront take part.
+__device__ __forceinline__ int slice_row_of(int rowoff, int nr, int q)
+{
+  int lo = 0;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1)
+  {
+    const int m = lo + o, v = __shfl(rowoff, min(m, 63), 64);
+    if (m < nr && v <= q) lo = m;
+  }
+  return lo;
+}
+
+// off-diagonal blocks W_ij = h s_i s_j H_i^b iM_b H_j^b' (ldy.c:738-844).  One
+// wavefront per slice, one lane per block, so that the stores are coalesced and
+// no lane waits for a longer row.  The block of a pair is formed with the lower
+// contact index as the "upper" side and transposed for the other, as the
+// reference's symmetry copy (ldy.c:830-844).  The rest of the last slot is
+// cleared: the sweeps load it.
 __global__ __launch_bounds__(TPB) void k_offdiag(BodyView bv, ConView cv, SellOut so, const int *perm,
                                                   const int *iperm, const int *rowptr, const int *col,
                                                   const int *via, int nslices, double step)
 {
-  int s = blockIdx.x*(TPB/SLICE) + (threadIdx.x >> 6), l = threadIdx.x & 63, r = l / G, g = l % G;
-  if (s >= nslices || r >= so.nrows[s]) return;
-  int p = so.row0[s] + r, i = perm[p];
-  long long off = so.off[s];
-  double *Wb = so.W + 9*off + l;
-  int *cb = so.wcol + off + l;
-  for (int k = g, m = 0; k < rowptr[i + 1] - rowptr[i]; k += G, m ++)
+  const int s = blockIdx.x*(TPB/SLICE) + (threadIdx.x >> 6), l = threadIdx.x & 63;
+  if (s >= nslices) return;
+  const int row0 = so.row0[s], nr = so.nrows[s], total = so.slen[s], ro = l < nr ? so.rowoff[row0 + l] : 0;
+  const long long off = so.off[s];
+  for (int q0 = 0; q0 < total; q0 += SLICE)
   {
-    int q = rowptr[i] + k, j = col[q], b = via[q];
+    const int k = q0 + l, r = slice_row_of(ro, nr, k), first = __shfl(ro, r, 64);
+    double *Wb = so.W + 9*(off + q0) + l;
+    if (k >= total)
+    {
+#pragma unroll
+      for (int e = 0; e < 9; e ++) Wb[e*SLICE] = 0.0;
+      so.wcol[off + k] = 0;
+      continue;
+    }
+    int i = perm[row0 + r], q = rowptr[i] + (k - first), j = col[q], b = via[q];
     int lo = i < j ? i : j, hi = i < j ? j : i;
     double sl = cv.master[lo] == b ? 1.0 : -1.0, sh = cv.master[hi] == b ? 1.0 : -1.0;
     const double *xl = sl > 0.0 ? cv.mpnt + 3*(size_t)lo : cv.spnt + 3*(size_t)lo;
@@ -536,20 +559,12 @@ __global__ __launch_bounds__(TPB) void k_offdiag(BodyView bv, ConView cv, SellOu
     operator_Hr(bv.rot + 9*(size_t)b, bv.x0 + 3*(size_t)b, xh, bh, Hh);
     h_im_ht(Hl, bl, Hh, bh, bv.jinv + 9*(size_t)b, bv.minv[b], P);
     double f = step * sl * sh;
-    if (i == lo)
-    {
+    const bool up = i == lo;
 #pragma unroll
-      for (int e = 0; e < 9; e ++) Wb[(9*(size_t)m + e)*SLICE] = f * P[e];
-    }
-    else
-    {
+    for (int rr = 0; rr < 3; rr ++)
 #pragma unroll
-      for (int rr = 0; rr < 3; rr ++)
-#pragma unroll
-        for (int c = 0; c < 3; c ++)
-          Wb[(9*(size_t)m + rr + 3*c)*SLICE] = f * P[c + 3*rr];
-    }
-    cb[(size_t)m*SLICE] = iperm[j];
+      for (int c = 0; c < 3; c ++) Wb[(rr + 3*c)*SLICE] = f * (up ? P[rr + 3*c] : P[c + 3*rr]);
+    so.wcol[off + k] = iperm[j];
   }
 }
 
@@ -589,21 +604,21 @@ __global__ __launch_bounds__(TPB) void k_rows_sys(SysIn si, RowsOut o, const int
   o.rowlen[p] = si.rowptr[i + 1] - si.rowptr[i];
 }
 
-template <int G>
 __global__ __launch_bounds__(TPB) void k_offdiag_sys(SysIn si, SellOut so, const int *perm, const int *iperm, int nslices)
 {
-  int s = blockIdx.x*(TPB/SLICE) + (threadIdx.x >> 6), l = threadIdx.x & 63, r = l / G, g = l % G;
-  if (s >= nslices || r >= so.nrows[s]) return;
-  int p = so.row0[s] + r, i = perm[p];
-  long long off = so.off[s];
-  double *Wb = so.W + 9*off + l;
-  int *cb = so.wcol + off + l;
-  for (int k = g, m = 0; k < si.rowptr[i + 1] - si.rowptr[i]; k += G, m ++)
+  const int s = blockIdx.x*(TPB/SLICE) + (threadIdx.x >> 6), l = threadIdx.x & 63;
+  if (s >= nslices) return;
+  const int row0 = so.row0[s], nr = so.nrows[s], total = so.slen[s], ro = l < nr ? so.rowoff[row0 + l] : 0;
+  const long long off = so.off[s];
+  for (int q0 = 0; q0 < total; q0 += SLICE)
   {
-    int q = si.rowptr[i] + k;
+    const int k = q0 + l, r = slice_row_of(ro, nr, k), first = __shfl(ro, r, 64);
+    const bool on = k < total;
+    const int q = on ? si.rowptr[perm[row0 + r]] + (k - first) : 0;
+    double *Wb = so.W + 9*(off + q0) + l;
 #pragma unroll
-    for (int e = 0; e < 9; e ++) Wb[(9*(size_t)m + e)*SLICE] = si.W[9*(size_t)q + e];
-    cb[(size_t)m*SLICE] = iperm[si.col[q]];
+    for (int e = 0; e < 9; e ++) Wb[e*SLICE] = on ? si.W[9*(size_t)q + e] : 0.0;
+    so.wcol[off + k] = on ? iperm[si.col[q]] : 0;
   }
 }
 
@@ -632,9 +647,10 @@ __global__ __launch_bounds__(WPB*64) void k_sweep(SweepArgs<T> a, int s0, int s1
   const int done = a.ctrl->done;
   const int bb = xcd ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
   const int s = s0 + bb*WPB + (threadIdx.x >> 6);
+  __shared__ T lds[WPB][MERIT ? Gather<T>::LDS2 : Gather<T>::LDS1];
   double eu = 0.0, el = 0.0, up = 0.0;
   sweep_slice<T, G, MERIT>(a, s, s < s1, upd_lo, upd_hi, backward, &a.ctrl->sweeps, a.failkey, a.failcount,
-                           &a.ctrl->aborted, eu, el, up, done == 0);
+                           &a.ctrl->aborted, eu, el, up, lds[threadIdx.x >> 6], done == 0);
   if (done) return;
   block_sum3<WPB*64>(eu, el, up);
   if (threadIdx.x == 0)
@@ -680,12 +696,13 @@ __global__ __launch_bounds__(NW*64) void k_sweep_group(SweepArgs<T> a, ColourGro
 {
   const int done = a.ctrl->done;
   const int w = threadIdx.x >> 6;
+  __shared__ T lds[NW][MERIT ? Gather<T>::LDS2 : Gather<T>::LDS1];
   double eu = 0.0, el = 0.0, up = 0.0;
   for (int q = 0; q < cg.n; q ++)
   {
     for (int s = cg.s0[q] + w; s < cg.s1[q]; s += NW)
       sweep_slice<T, G, MERIT>(a, s, true, cg.lo[q], cg.hi[q], backward, &a.ctrl->sweeps, a.failkey, a.failcount,
-                               &a.ctrl->aborted, eu, el, up, done == 0);
+                               &a.ctrl->aborted, eu, el, up, lds[w], done == 0);
     __syncthreads();   // this colour's reactions before the next colour's gathers
   }
   if (done) return;
@@ -708,8 +725,9 @@ template <int G>
 __global__ __launch_bounds__(TPB) void k_merit(MeritArgs a, int nslices)
 {
   const int s = blockIdx.x*(TPB/SLICE) + (threadIdx.x >> 6);
+  __shared__ double lds[TPB/SLICE][Gather<double>::LDS1];
   double up = 0.0, z1 = 0.0, z2 = 0.0;
-  merit_slice<G>(a, s, s < nslices, up);
+  merit_slice<G>(a, s, s < nslices, up, lds[threadIdx.x >> 6]);
   block_sum3(up, z1, z2);
   if (threadIdx.x == 0) a.mpartials[blockIdx.x] = up;
 }
@@ -1233,6 +1251,7 @@ static int build_order(sfgs_ctx *ctx, int n, bool have_master)
   CHK(ensure(ctx, ctx->svals, n));
   CHK(ensure(ctx, ctx->perm, n));
   CHK(ensure(ctx, ctx->iperm, n));
+  CHK(ensure(ctx, ctx->rowoff, n));
   // orders 2 and 3 need the master bodies of the contacts (a system uploaded as W has none)
   const int mode = ctx->row_order >= 2 && !have_master ? 0 : ctx->row_order;
   int keybits = mode >= 2 ? 40 : 32;
@@ -1305,8 +1324,8 @@ static int build_order(sfgs_ctx *ctx, int n, bool have_master)
   CHK(ensure(ctx, lens, (size_t)ns + 1));
   HIPCHK(hipMemsetAsync(lens.p, 0, sizeof(long long)*((size_t)ns + 1), ctx->stream));
   if (ns > 0)
-    hipLaunchKernelGGL(k_slice_len, dim3(nblk(ns)), dim3(TPB), 0, ctx->stream, ns, ctx->slice_row0.p, ctx->slice_nrows.p, ctx->perm.p,
-                       ctx->rowptr.p, G, ctx->slice_len.p, lens.p);
+    hipLaunchKernelGGL(k_slice_len, dim3(nblk((long long)ns*SLICE)), dim3(TPB), 0, ctx->stream, ns, ctx->slice_row0.p,
+                       ctx->slice_nrows.p, ctx->perm.p, ctx->rowptr.p, ctx->rowoff.p, ctx->slice_len.p, lens.p);
   CHK(scan_ll(ctx, lens.p, ctx->slice_off.p, ns + 1));
   long long total = 0;
   HIPCHK(hipMemcpyAsync(&total, ctx->slice_off.p + ns, sizeof(long long), hipMemcpyDeviceToHost, ctx->stream));
@@ -1315,11 +1334,6 @@ static int build_order(sfgs_ctx *ctx, int n, bool have_master)
   ctx->sell_blocks = total;
   CHK(ensure(ctx, ctx->W, (size_t)(9*total)));
   CHK(ensure(ctx, ctx->wcol, (size_t)total));
-  if (total > 0)
-  {
-    HIPCHK(hipMemsetAsync(ctx->W.p, 0, sizeof(double)*(size_t)(9*total), ctx->stream));
-    HIPCHK(hipMemsetAsync(ctx->wcol.p, 0, sizeof(int)*(size_t)total, ctx->stream));
-  }
   return 0;
 }
 
@@ -1389,6 +1403,7 @@ static SellOut sell_out(sfgs_ctx *ctx)
 {
   SellOut so;
   so.row0 = ctx->slice_row0.p; so.nrows = ctx->slice_nrows.p; so.off = ctx->slice_off.p;
+  so.rowoff = ctx->rowoff.p; so.slen = ctx->slice_len.p;
   so.W = ctx->W.p; so.wcol = ctx->wcol.p;
   return so;
 }
@@ -1483,7 +1498,7 @@ void SFGS_Destroy(sfgs_ctx *ctx)
   release(ctx->colour); release(ctx->colour2); release(ctx->perm); release(ctx->iperm); release(ctx->counter);
   release(ctx->skeys); release(ctx->skeys2); release(ctx->svals); release(ctx->svals2); release(ctx->scratch); release(ctx->bbox);
   release(ctx->slice_row0); release(ctx->slice_nrows); release(ctx->slice_len); release(ctx->slice_off);
-  release(ctx->rowlen); release(ctx->W); release(ctx->Wd); release(ctx->A); release(ctx->B); release(ctx->V);
+  release(ctx->rowlen); release(ctx->rowoff); release(ctx->W); release(ctx->Wd); release(ctx->A); release(ctx->B); release(ctx->V);
   release(ctx->rho); release(ctx->pfri); release(ctx->pcoh); release(ctx->shift); release(ctx->R); release(ctx->U); release(ctx->pen); sfgs_newton_release(ctx); sfgs_bar_release(ctx);
   release(ctx->Rb); release(ctx->Um); release(ctx->sep); release(ctx->wcol);
   release(ctx->W32); release(ctx->Wd32); release(ctx->rec32); release(ctx->B32); release(ctx->R32); release(ctx->R32b); release(ctx->U32); release(ctx->Um32);
@@ -1638,9 +1653,8 @@ static int locdyn_update(sfgs_ctx *ctx, double step, int dynamic, bool full)
     hipLaunchKernelGGL(k_rows, dim3(nbk), dim3(TPB), 0, st, bv, cv, rows_out(ctx, nc, ctx->partials.p, ctx->failcount.p),
                        ctx->perm.p, ctx->rowptr.p, step, dynamic);
     if (ctx->nslices > 0)
-      SFGS_DISPATCH_G(ctx->G_built, auto kern = k_offdiag<GG>; hipLaunchKernelGGL(kern, dim3(nblk((long long)ctx->nslices*SLICE)), dim3(TPB),
-                      0, st, bv, cv, sell_out(ctx), ctx->perm.p, ctx->iperm.p, ctx->rowptr.p, ctx->col.p, ctx->via.p,
-                      ctx->nslices, step));
+      hipLaunchKernelGGL(k_offdiag, dim3(nblk((long long)ctx->nslices*SLICE)), dim3(TPB), 0, st, bv, cv, sell_out(ctx),
+                         ctx->perm.p, ctx->iperm.p, ctx->rowptr.p, ctx->col.p, ctx->via.p, ctx->nslices, step);
   }
   std::vector<double> ep((size_t)std::max(nbk, 1), 0.0);
   int singular = 0;
@@ -1713,8 +1727,8 @@ int SFGS_System_Upload(sfgs_ctx *ctx, int n, const int *rowptr, const int *col, 
     hipLaunchKernelGGL(k_rows_sys, dim3(nblk(n)), dim3(TPB), 0, st, si, rows_out(ctx, n, nullptr, nullptr),
                        ctx->perm.p, step, dynamic);
     if (ctx->nslices > 0)
-      SFGS_DISPATCH_G(ctx->G_built, auto kern = k_offdiag_sys<GG>; hipLaunchKernelGGL(kern, dim3(nblk((long long)ctx->nslices*SLICE)),
-                      dim3(TPB), 0, st, si, sell_out(ctx), ctx->perm.p, ctx->iperm.p, ctx->nslices));
+      hipLaunchKernelGGL(k_offdiag_sys, dim3(nblk((long long)ctx->nslices*SLICE)), dim3(TPB), 0, st, si, sell_out(ctx),
+                         ctx->perm.p, ctx->iperm.p, ctx->nslices);
   }
   hipError_t e = hipStreamSynchronize(st);
   release(dW); release(dWd); release(dA); release(dB); release(dV); release(drho); release(dfri);
@@ -2456,17 +2470,14 @@ int SFGS_Get_Locdyn(sfgs_ctx *ctx, int *rowptr, int *col, int *via, double *W, d
   }
   if (W)
   {
-    // SELL slot k of row p holds the k-th block of the natural row perm[p]
+    // the blocks of a slice are those of its rows, one natural row after the other
     for (int s = 0; s < ctx->nslices; s ++)
-      for (int l = 0; l < hnr[s]; l ++)
+      for (int l = 0, k = 0; l < hnr[s]; l ++)
       {
         int p = hrow0[s] + l, i = hperm[p];
-        for (int q = hrowptr[i], k = 0; q < hrowptr[i + 1]; q ++, k ++)
-        {
-          int G = ctx->G_built, m = k / G, lane = l*G + k % G;
+        for (int q = hrowptr[i]; q < hrowptr[i + 1]; q ++, k ++)
           for (int e = 0; e < 9; e ++)
-            W[9*(size_t)q + e] = hW[9*(size_t)hoff[s] + (9*(size_t)m + e)*SLICE + lane];
-        }
+            W[9*(size_t)q + e] = hW[9*(size_t)hoff[s] + (9*(size_t)(k / SLICE) + e)*SLICE + k % SLICE];
       }
   }
   return 0;

@@ -109,7 +109,7 @@ __global__ __launch_bounds__(TPB) void k_nt_lin(NtRows a, int diag, double omega
 }
 
 struct NtMat {
-  const int *row0, *nrows, *rowlen;
+  const int *row0, *nrows, *rowlen, *rowoff, *slen;
   const long long *off;
   const double *W;
   const int *wcol;
@@ -122,25 +122,16 @@ template <int G>
 __global__ __launch_bounds__(TPB) void k_nt_matvec(NtMat a, int nslices, double alpha, const double *x, double beta,
                                                     double *y)
 {
-  const int s = blockIdx.x*(TPB/SLICE) + (threadIdx.x >> 6);
-  if (s >= nslices) return;   // uniform over the wavefront
+  const int sl = blockIdx.x*(TPB/SLICE) + (threadIdx.x >> 6);
+  if (sl >= nslices) return;   // uniform over the wavefront
   const int l = threadIdx.x & 63, r = l / G, g = l % G, n = a.n;
+  const int s = __builtin_amdgcn_readfirstlane(sl);
   const bool act = r < a.nrows[s];
-  const long long off = a.off[s];
-  const int p = a.row0[s] + r, len = act ? a.rowlen[p] : 0;
-  double z0 = 0.0, z1 = 0.0, z2 = 0.0;
-  const double *Wb = a.W + 9*off + l;
-  const int *cb = a.wcol + off + l;
-  for (int k = g, m = 0; k < len; k += G, m ++)
-  {
-    const int j = cb[(size_t)m*SLICE];
-    const double *w = Wb + 9*(size_t)m*SLICE;
-    const double x0 = x[3*(size_t)j], x1 = x[3*(size_t)j + 1], x2 = x[3*(size_t)j + 2];
-    z0 += w[0]*x0 + w[3*SLICE]*x1 + w[6*SLICE]*x2;
-    z1 += w[SLICE]*x0 + w[4*SLICE]*x1 + w[7*SLICE]*x2;
-    z2 += w[2*SLICE]*x0 + w[5*SLICE]*x1 + w[8*SLICE]*x2;
-  }
-  z0 = gsum<G>(z0); z1 = gsum<G>(z1); z2 = gsum<G>(z2);
+  const int p = a.row0[s] + (act ? r : 0), len = a.rowlen[p], rs = a.rowoff[p];
+  __shared__ double lds[TPB/SLICE][Gather<double>::LDS1];
+  double zz[3], none[3];
+  gather_rows<double, G, false, false, 3>(a.W, a.wcol, a.off[s], a.slen[s], rs, len, act, x, x, 0, 0, lds[threadIdx.x >> 6],
+                                          zz, none);
   if (!act || g != 0) return;
   const double xp[3] = {x[3*(size_t)p], x[3*(size_t)p + 1], x[3*(size_t)p + 2]};
   double Wi[9], X[9], Y[9];
@@ -151,9 +142,9 @@ __global__ __launch_bounds__(TPB) void k_nt_matvec(NtMat a, int nslices, double 
     X[e] = a.X[(size_t)e*n + p];
     Y[e] = a.Y[(size_t)e*n + p];
   }
-  const double z[3] = {Wi[0]*xp[0] + Wi[3]*xp[1] + Wi[6]*xp[2] + z0,
-                       Wi[1]*xp[0] + Wi[4]*xp[1] + Wi[7]*xp[2] + z1,
-                       Wi[2]*xp[0] + Wi[5]*xp[1] + Wi[8]*xp[2] + z2};
+  const double z[3] = {Wi[0]*xp[0] + Wi[3]*xp[1] + Wi[6]*xp[2] + zz[0],
+                       Wi[1]*xp[0] + Wi[4]*xp[1] + Wi[7]*xp[2] + zz[1],
+                       Wi[2]*xp[0] + Wi[5]*xp[1] + Wi[8]*xp[2] + zz[2]};
   const double ad = alpha*a.delta;
 #pragma unroll
   for (int k = 0; k < 3; k ++)
@@ -518,8 +509,8 @@ int SFGS_Newton_Solve(sfgs_ctx *ctx, const SFGS_NEWTON_PARAM *par, double *merhi
   else if (par->reldelta == 3) W_norm = 0.0;
   const double delta = par->delta*W_norm;
 
-  wk.mat = NtMat{ctx->slice_row0.p, ctx->slice_nrows.p, ctx->rowlen.p, ctx->slice_off.p, ctx->W.p, ctx->wcol.p,
-                 ctx->Wd.p, wk.X, wk.Y, n, delta};
+  wk.mat = NtMat{ctx->slice_row0.p, ctx->slice_nrows.p, ctx->rowlen.p, ctx->rowoff.p, ctx->slice_len.p,
+                 ctx->slice_off.p, ctx->W.p, ctx->wcol.p, ctx->Wd.p, wk.X, wk.Y, n, delta};
   NtRows rows{n, ctx->R.p, ctx->U.p, ctx->Wd.p, ctx->pfri.p, ctx->pcoh.p, ctx->shift.p, wk.X, wk.Y, wk.P, wk.b, wk.dr,
               ctx->failcount.p};
 

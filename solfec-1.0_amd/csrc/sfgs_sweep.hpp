@@ -40,7 +40,8 @@ __device__ __forceinline__ T wave_sum(T v)
 template <typename T>
 struct SweepArgs {
   const int *row0, *nrows, *rowlen;
-  const int *slen;      // block slots per lane of each slice (those of its first, longest row)
+  const int *rowoff;    // first block of each row in its slice
+  const int *slen;      // blocks of each slice
   const long long *off;
   const T *W;
   const int *wcol;
@@ -109,6 +110,152 @@ __device__ __forceinline__ void r_st(T *p, T v)
   else *p = v;
 }
 
+// ---- the gather of a slice: sum_j W_ij x_j of its rows ----
+//
+// The blocks of a slice are stored row after row without gaps, block q in lane
+// q mod 64 of slot q / 64, so a wavefront reads them one per lane whatever the
+// rows' lengths: no padding but in the last slot (the slices of a 200k packing
+// were one third padding with a fixed number of slots per row), every load full,
+// and few load instructions, which is what this phase is bound by: a slice of 32
+// rows with 7.4 blocks each takes 4 slots of 9 + 1 coalesced loads and a gather of
+// 16-byte reactions.  Each lane forms its block's product and leaves it in LDS;
+// then the G lanes of a row add the row's products, lane g those of blocks g,
+// g + G, ..., in that order, so that the sums do not depend on the layout.
+// CS slots are in flight together, the indices ahead of the blocks and nothing
+// else waited for (straight-line code per number of slots: branches around single
+// slots, or zeros merged into a lane without a row, cost a wait each and made this
+// slower than the padded layout).  A slice with more slots goes round again; six
+// (FP32) and four (FP64) hold most slices in one round within the registers of
+// three and two wavefronts per SIMD.  1000 mixed sweeps of a 200k-sphere packing
+// (417k rows): the whole step 158.5 -> 135.4 ms, 500 FP64 ones 138.7 -> 126.6 ms,
+// 64 scenes of 628k rows, 300 mixed sweeps, 84.6 -> 72.6 ms; clock cycles of this
+// phase in a large colour 14-16k -> 9-11k (FP32), 22-37k -> 13k (FP64).
+template <typename T> struct Gather {
+  static const int CS = sizeof(T) == 8 ? 4 : 6;   // slots in flight
+  static const int CB = CS*SLICE;
+  static const int LDS2 = 6*CB, LDS1 = 3*CB;      // LDS values per wavefront: two products of a block, or one
+};
+
+// reaction (or other 3-vector) j at x + S j: 16-byte loads where the stride keeps them aligned
+template <bool COH, int S, typename T>
+__device__ __forceinline__ void load3(const T *x, int j, T (&v)[3])
+{
+  const T *p = x + (size_t)S*j;
+  if constexpr (!COH && S == 4 && sizeof(T) == 4)
+  {
+    const float4 q = *reinterpret_cast<const float4 *>(p);
+    v[0] = q.x; v[1] = q.y; v[2] = q.z;
+  }
+  else if constexpr (!COH && S == 4)
+  {
+    const double2 q = *reinterpret_cast<const double2 *>(p);
+    v[0] = q.x; v[1] = q.y; v[2] = p[2];
+  }
+  else { v[0] = r_ld<COH>(p); v[1] = r_ld<COH>(p + 1); v[2] = r_ld<COH>(p + 2); }
+}
+
+__device__ __forceinline__ void wave_lds_fence()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// N slots: each lane's block times its reaction(s), into d[c CB + 64 q] (slot q)
+template <typename T, int N, bool TWO, bool COH, int S>
+__device__ __forceinline__ void gather_slots(const T *W, const int *cb, const T *P, const T *Q, int upd_lo, int upd_hi,
+                                             T *d)
+{
+  constexpr int CB = Gather<T>::CB;
+  int jj[N];
+  T wv[N][9], rv[N][3], pv[N][3];
+#pragma unroll
+  for (int q = 0; q < N; q ++) jj[q] = cb[q*SLICE];
+#pragma unroll
+  for (int q = 0; q < N; q ++)
+#pragma unroll
+    for (int e = 0; e < 9; e ++) wv[q][e] = W[(9*q + e)*SLICE];
+  // the block loads ahead of the first wait for the indices
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int q = 0; q < N; q ++)
+  {
+    const int j = jj[q];
+    load3<COH, S>(j >= upd_lo && j < upd_hi ? Q : P, j, rv[q]);
+    if (TWO) load3<COH, S>(P, j, pv[q]);
+  }
+#pragma unroll
+  for (int q = 0; q < N; q ++)
+#pragma unroll
+    for (int c = 0; c < 3; c ++)
+    {
+      // explicit fused multiply-adds: the same rounding wherever this is inlined
+      d[c*CB + q*SLICE] = fma(wv[q][6 + c], rv[q][2], fma(wv[q][3 + c], rv[q][1], wv[q][c]*rv[q][0]));
+      if (TWO) d[(3 + c)*CB + q*SLICE] = fma(wv[q][6 + c], pv[q][2], fma(wv[q][3 + c], pv[q][1], wv[q][c]*pv[q][0]));
+    }
+}
+
+// sums b of W_ij (upd ? Q : P)_j over the row's blocks and, when TWO, u of
+// W_ij P_j.  off and total (wave-uniform): the slice's first block slot and its
+// number of blocks; rs, len: the row's first block and their number and
+// whether the lane has a row.  The sums over the G lanes are complete on return.
+template <typename T, int G, bool TWO, bool COH, int S>
+__device__ __forceinline__ void gather_rows(const T *W, const int *wcol, long long off, int total, int rs, int len,
+                                            bool act, const T *P, const T *Q, int upd_lo, int upd_hi, T *lds,
+                                            T (&b)[3], T (&u)[3])
+{
+  constexpr int CS = Gather<T>::CS, CB = Gather<T>::CB;
+  const int l = threadIdx.x & 63, g = l % G, ns = (total + SLICE - 1) / SLICE;
+  const T *Wb = W + 9*off + l;
+  const int *cb = wcol + off + l;
+#pragma unroll
+  for (int c = 0; c < 3; c ++) b[c] = u[c] = T(0);
+  int k = g;
+  for (int m0 = 0; m0 < ns; m0 += CS)
+  {
+    const T *Wm = Wb + 9*m0*SLICE;
+    const int *cm = cb + m0*SLICE;
+    // straight-line code per number of slots: all loads of a round in flight
+    switch (min(ns - m0, CS))
+    {
+    case 1: gather_slots<T, 1, TWO, COH, S>(Wm, cm, P, Q, upd_lo, upd_hi, lds + l); break;
+    case 2: gather_slots<T, 2, TWO, COH, S>(Wm, cm, P, Q, upd_lo, upd_hi, lds + l); break;
+    case 3: gather_slots<T, 3, TWO, COH, S>(Wm, cm, P, Q, upd_lo, upd_hi, lds + l); break;
+    case 4: gather_slots<T, 4, TWO, COH, S>(Wm, cm, P, Q, upd_lo, upd_hi, lds + l); break;
+    case 5: if constexpr (CS >= 5) gather_slots<T, 5, TWO, COH, S>(Wm, cm, P, Q, upd_lo, upd_hi, lds + l); break;
+    default: if constexpr (CS >= 6) gather_slots<T, 6, TWO, COH, S>(Wm, cm, P, Q, upd_lo, upd_hi, lds + l); break;
+    }
+    wave_lds_fence();
+    // rs and len may still be in flight: not used, nor hoisted, before here
+    int rr = rs, ln = len;
+    asm volatile("" : "+v"(rr), "+v"(ln));
+    const int end = act ? min(ln, m0*SLICE + CB - rr) : 0, base = rr - m0*SLICE;
+    for (; k < end; k += 4*G)
+    {
+      T t[4][6];
+#pragma unroll
+      for (int q = 0; q < 4; q ++)
+      {
+        const T *d = lds + base + min(k + q*G, end - 1);
+#pragma unroll
+        for (int c = 0; c < (TWO ? 6 : 3); c ++) t[q][c] = d[c*CB];
+      }
+#pragma unroll
+      for (int q = 0; q < 4; q ++)
+        if (k + q*G < end)
+        {
+#pragma unroll
+          for (int c = 0; c < 3; c ++) { b[c] += t[q][c]; if (TWO) u[c] += t[q][3 + c]; }
+        }
+    }
+    // the last round may have stepped past the chunk: back to the lane's first block beyond it
+    if (k > end) k = end > g ? g + (end - g + G - 1)/G*G : g;
+    wave_lds_fence();
+  }
+#pragma unroll
+  for (int c = 0; c < 3; c ++) { b[c] = gsum<G>(b[c]); if (TWO) u[c] = gsum<G>(u[c]); }
+}
+
 // One slice (64/G rows of one colour, one wavefront) of a sweep.  eu, el and
 // up receive this lane's contributions to the error sums and to the merit
 // numerator.  A failed local solve is recorded in failkey / failcount, keyed by
@@ -116,151 +263,89 @@ __device__ __forceinline__ void r_st(T *p, T v)
 // false (a solve that has stopped) leaves the slice untouched; the caller reads
 // that flag together with the slice table, so both cost one memory round trip.
 // COH: P and Q are shared with other wavefronts of the same launch (r_ld / r_st).
+// lds: this wavefront's Gather<T>::LDS2 (merit) or LDS1 values.  s and valid are
+// the same in all lanes of the wavefront.
 template <typename T, int G, bool MERIT, bool COH = false>
 __device__ __forceinline__ void sweep_slice(const SweepArgs<T> &a, int s, bool valid, int upd_lo, int upd_hi,
                                             int backward, const int *sweepno, unsigned long long *failkey,
                                             int *failcount, int *abortflag, double &eu, double &el, double &up,
-                                            bool run = true)
+                                            T *lds, bool run = true)
 {
   const int l = threadIdx.x & 63, r = l / G, g = l % G;
   const int n = a.n;
-  int nr = 0, r0 = 0, p = 0, len = 0;
-  long long off = 0;
-  if (valid) { nr = a.nrows[s]; r0 = a.row0[s]; off = a.off[s]; }   // one round of loads
-  const bool act = valid && run && r < nr;
-  // the row's own data first, so that its loads overlap the gather below
-  T Bi[3] = {T(0), T(0), T(0)}, Wi[9], R[3] = {T(0), T(0), T(0)}, U[3] = {T(0), T(0), T(0)};
-  double Ai[9];
-  RowLaw<T> L{T(0), T(0), T(0), T(0), false};
+  s = __builtin_amdgcn_readfirstlane(s);
+  if (!__builtin_amdgcn_readfirstlane(valid && run)) return;
+  const int nr = a.nrows[s], r0 = a.row0[s], total = a.slen[s];   // one round of loads
+  const long long off = a.off[s];
+  const bool act = r < nr;
+  // The row's own data first, so that its loads are in flight with the gather's.
+  // Nothing is computed from them before the gather (a use waits for them), and
+  // lanes without a row load the last one's (so would a merge of two paths).
+  const int p = r0 + min(r, nr - 1), rs = a.rowoff[p], len = a.rowlen[p];
+  T Bi[3], Wi[9], R[3], U[3], A64[9];
+  float4 rec[5];
+  RowLaw<T> L;
+  unsigned char sep = 0;
+  if constexpr (sizeof(T) == 4)
+  {
+    // the row record: five 16-byte loads (k_rec32)
+#pragma unroll
+    for (int k = 0; k < 5; k ++) rec[k] = a.rec[5*(size_t)p + k];
+  }
+  else
+  {
+    Bi[0] = a.B[p]; Bi[1] = a.B[(size_t)n + p]; Bi[2] = a.B[2*(size_t)n + p];
+#pragma unroll
+    for (int e = 0; e < 9; e ++) Wi[e] = a.Wd[(size_t)e*n + p];
+    if (MERIT)
+    {
+#pragma unroll
+      for (int e = 0; e < 9; e ++) A64[e] = a.A[(size_t)e*n + p];
+    }
+    L = RowLaw<T>{a.fri[p], a.coh[p], a.shift[p], a.rho[p], false};
+    sep = a.sep[p];
+  }
+  load3<COH, 4>(a.P, p, R);
+  if (!MERIT)
+  {
+#pragma unroll
+    for (int k = 0; k < 3; k ++) U[k] = a.Uin[(size_t)k*n + p];
+  }
+  T b[3], u[3];
+  gather_rows<T, G, MERIT, COH, 4>(a.W, a.wcol, off, total, rs, len, act, a.P, a.Q, upd_lo, upd_hi, lds, b, u);
+
   if (act)
   {
-    p = r0 + r;
+    double Ai[9];
     if constexpr (sizeof(T) == 4)
     {
-      // the row record: five 16-byte loads (k_rec32), and R_i as one when not shared
-      const float4 *rc = a.rec + 5*(size_t)p;
-      const float4 q0 = rc[0], q1 = rc[1], q2 = rc[2], q3 = rc[3], q4 = rc[4];
-      const int ls = __float_as_int(q1.w);
-      len = ls >> 1;
-      Bi[0] = q0.x; Bi[1] = q0.y; Bi[2] = q0.z;
-      Wi[0] = q2.x; Wi[1] = Wi[3] = q2.y; Wi[2] = Wi[6] = q2.z; Wi[4] = q2.w; Wi[5] = Wi[7] = q3.x; Wi[8] = q3.y;
+      Bi[0] = rec[0].x; Bi[1] = rec[0].y; Bi[2] = rec[0].z;
+      const int ls = __float_as_int(rec[1].w);
+      L = RowLaw<T>{rec[1].x, rec[1].y, rec[1].z, rec[0].w, (ls & 1) != 0};
+      Wi[0] = rec[2].x; Wi[1] = Wi[3] = rec[2].y; Wi[2] = Wi[6] = rec[2].z; Wi[4] = rec[2].w;
+      Wi[5] = Wi[7] = rec[3].x; Wi[8] = rec[3].y;
       if (MERIT)
       {
-        Ai[0] = q3.z; Ai[1] = Ai[3] = q3.w; Ai[2] = Ai[6] = q4.x; Ai[4] = q4.y; Ai[5] = Ai[7] = q4.z; Ai[8] = q4.w;
-      }
-      L = RowLaw<T>{q1.x, q1.y, q1.z, q0.w, (ls & 1) != 0};
-      if (COH)
-      {
-#pragma unroll
-        for (int k = 0; k < 3; k ++) R[k] = r_ld<COH>(a.P + 4*(size_t)p + k);
-      }
-      else
-      {
-        const float4 rr = *reinterpret_cast<const float4 *>(a.P + 4*(size_t)p);
-        R[0] = rr.x; R[1] = rr.y; R[2] = rr.z;
+        Ai[0] = rec[3].z; Ai[1] = Ai[3] = rec[3].w; Ai[2] = Ai[6] = rec[4].x;
+        Ai[4] = rec[4].y; Ai[5] = Ai[7] = rec[4].z; Ai[8] = rec[4].w;
       }
     }
     else
     {
-      len = a.rowlen[p];
-      Bi[0] = a.B[p]; Bi[1] = a.B[(size_t)n + p]; Bi[2] = a.B[2*(size_t)n + p];
-#pragma unroll
-      for (int e = 0; e < 9; e ++) Wi[e] = a.Wd[(size_t)e*n + p];
-#pragma unroll
-      for (int k = 0; k < 3; k ++) R[k] = r_ld<COH>(a.P + 4*(size_t)p + k);
+      L.separated = sep != 0;
       if (MERIT)
       {
 #pragma unroll
-        for (int e = 0; e < 9; e ++) Ai[e] = a.A[(size_t)e*n + p];
-      }
-      L = RowLaw<T>{a.fri[p], a.coh[p], a.shift[p], a.rho[p], a.sep[p] != 0};
-    }
-    if (!MERIT)
-    {
-#pragma unroll
-      for (int k = 0; k < 3; k ++) U[k] = a.Uin[(size_t)k*n + p];
-    }
-  }
-  T b0 = T(0), b1 = T(0), b2 = T(0), u0 = T(0), u1 = T(0), u2 = T(0);
-  if (act)
-  {
-    // The gather runs over the slice's slot count, known with the slice table,
-    // so the neighbour indices and blocks load without waiting for this row's
-    // length; slots past the row's own (padding: zero block, row 0) are loaded
-    // but not added.  CH slots at a time: all their indices, then all their
-    // blocks and reactions, in flight together.
-    constexpr int CH = sizeof(T) == 8 ? 4 : 8;
-    const T *Wb = a.W + 9*off + l;
-    const int *cb = a.wcol + off + l;
-    const int nsl = a.slen[s], mine = len > g ? (len - g + G - 1) / G : 0;
-    for (int m0 = 0; m0 < nsl; m0 += CH)
-    {
-      // branch-free: every load of the chunk is issued before any is waited for
-      // (slots past the slice's own re-read its last slot and are not added)
-      int jj[CH];
-#pragma unroll
-      for (int q = 0; q < CH; q ++) jj[q] = m0 + q < nsl ? cb[(size_t)(m0 + q)*SLICE] : 0;
-      // the blocks do not depend on the indices: issued with them, before any wait
-      T wv[CH][9], rv[CH][3], pv[CH][3];
-#pragma unroll
-      for (int q = 0; q < CH; q ++)
-      {
-        const int m = min(m0 + q, nsl - 1);
-        const T *w = Wb + 9*(size_t)m*SLICE;
-#pragma unroll
-        for (int e = 0; e < 9; e ++) wv[q][e] = w[e*SLICE];
-      }
-      // keep the block loads ahead of the first wait for the indices
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int q = 0; q < CH; q ++)
-      {
-        const int j = jj[q];
-        const bool upd = j >= upd_lo && j < upd_hi;
-        const T *xj = (upd ? a.Q : a.P) + 4*(size_t)j;
-        rv[q][0] = r_ld<COH>(xj); rv[q][1] = r_ld<COH>(xj + 1); rv[q][2] = r_ld<COH>(xj + 2);
-        if (MERIT)
-        {
-          // the previous iterate of every neighbour (equal to rv where not yet updated)
-          const T *pj = a.P + 4*(size_t)j;
-          pv[q][0] = r_ld<COH>(pj); pv[q][1] = r_ld<COH>(pj + 1); pv[q][2] = r_ld<COH>(pj + 2);
-        }
-      }
-#pragma unroll
-      for (int q = 0; q < CH; q ++)
-      {
-        const bool on = m0 + q < mine;
-        const T w0 = wv[q][0], w1 = wv[q][1], w2 = wv[q][2], w3 = wv[q][3], w4 = wv[q][4], w5 = wv[q][5],
-                w6 = wv[q][6], w7 = wv[q][7], w8 = wv[q][8];
-        const T r0 = rv[q][0], r1 = rv[q][1], r2 = rv[q][2];
-        // explicit fused multiply-adds: the same rounding in every schedule
-        // that instantiates this gather, whatever the surrounding loads
-        b0 = on ? b0 + fma(w6, r2, fma(w3, r1, w0*r0)) : b0;
-        b1 = on ? b1 + fma(w7, r2, fma(w4, r1, w1*r0)) : b1;
-        b2 = on ? b2 + fma(w8, r2, fma(w5, r1, w2*r0)) : b2;
-        if (MERIT)
-        {
-          const T p0 = pv[q][0], p1 = pv[q][1], p2 = pv[q][2];
-          u0 = on ? u0 + fma(w6, p2, fma(w3, p1, w0*p0)) : u0;
-          u1 = on ? u1 + fma(w7, p2, fma(w4, p1, w1*p0)) : u1;
-          u2 = on ? u2 + fma(w8, p2, fma(w5, p1, w2*p0)) : u2;
-        }
+        for (int e = 0; e < 9; e ++) Ai[e] = A64[e];
       }
     }
-  }
-  // sum over the G lanes of each row; every lane of the wave takes part
-  b0 = gsum<G>(b0); b1 = gsum<G>(b1); b2 = gsum<G>(b2);
-  if (MERIT) { u0 = gsum<G>(u0); u1 = gsum<G>(u1); u2 = gsum<G>(u2); }
-
-  if (act)
-  {
-    T Bp[3] = {Bi[0] + b0, Bi[1] + b1, Bi[2] + b2};
+    T Bp[3] = {Bi[0] + b[0], Bi[1] + b[1], Bi[2] + b[2]};
     const T R0[3] = {R[0], R[1], R[2]};
     if (MERIT)
     {
       // merit of the previous iteration at this row (mrf.c:63-84)
       mv_add(Bi, Wi, R, U);
-      U[0] += u0; U[1] += u1; U[2] += u2;
+      U[0] += u[0]; U[1] += u[1]; U[2] += u[2];
       // the merit is evaluated in FP64 whatever the sweep type
       double C[3], Ud[3] = {U[0], U[1], U[2]}, Rd[3] = {R[0], R[1], R[2]};
       scf_residual<double>(L.fri, L.coh, L.shift, Ud, Rd, C, nullptr, nullptr);
@@ -328,7 +413,7 @@ __device__ __forceinline__ void sweep_slice(const SweepArgs<T> &a, int s, bool v
 // standalone merit (MERIT_Function with update_U, mrf.c:35-184) on the
 // canonical R buffer; one launch over all slices
 struct MeritArgs {
-  const int *row0, *nrows, *rowlen;
+  const int *row0, *nrows, *rowlen, *rowoff, *slen;
   const long long *off;
   const double *W;
   const int *wcol;
@@ -340,38 +425,28 @@ struct MeritArgs {
   double *conmerit;   // may be null: per-row C'AC (colour-major)
 };
 
-// merit terms C'AC of the rows of one slice, added to up (lane g = 0 of each row)
+// merit terms C'AC of the rows of one slice, added to up (lane g = 0 of each
+// row); lds: this wavefront's Gather<double>::LDS1 values
 template <int G>
-__device__ __forceinline__ void merit_slice(const MeritArgs &a, int s, bool valid, double &up)
+__device__ __forceinline__ void merit_slice(const MeritArgs &a, int s, bool valid, double &up, double *lds)
 {
   const int l = threadIdx.x & 63, r = l / G, g = l % G;
   const int n = a.n;
-  bool act = false;
-  int p = 0, len = 0;
+  int nr = 0, r0 = 0, total = 0;
   long long off = 0;
-  if (valid)
+  s = __builtin_amdgcn_readfirstlane(s);
+  if (__builtin_amdgcn_readfirstlane(valid))
   {
-    act = r < a.nrows[s];
-    off = a.off[s];
-    if (act) { p = a.row0[s] + r; len = a.update_U ? a.rowlen[p] : 0; }
+    nr = a.nrows[s]; r0 = a.row0[s];
+    if (a.update_U) { off = a.off[s]; total = a.slen[s]; }
   }
-  double u0 = 0.0, u1 = 0.0, u2 = 0.0;
-  if (act)
-  {
-    const double *Wb = a.W + 9*off + l;
-    const int *cb = a.wcol + off + l;
-    for (int k = g, m = 0; k < len; k += G, m ++)
-    {
-      const int j = cb[(size_t)m*SLICE];
-      const double *w = Wb + 9*(size_t)m*SLICE;
-      const double r0 = a.R[4*(size_t)j], r1 = a.R[4*(size_t)j + 1], r2 = a.R[4*(size_t)j + 2];
-      // the sweep's multiply-adds (sweep_slice), so that U equals the fused merit pass's
-      u0 = u0 + fma(w[6*SLICE], r2, fma(w[3*SLICE], r1, w[0]*r0));
-      u1 = u1 + fma(w[7*SLICE], r2, fma(w[4*SLICE], r1, w[SLICE]*r0));
-      u2 = u2 + fma(w[8*SLICE], r2, fma(w[5*SLICE], r1, w[2*SLICE]*r0));
-    }
-  }
-  u0 = gsum<G>(u0); u1 = gsum<G>(u1); u2 = gsum<G>(u2);
+  const bool act = r < nr;
+  const int p = act ? r0 + r : 0;
+  int len = 0, rs = 0;
+  if (total > 0) { len = a.rowlen[p]; rs = a.rowoff[p]; }
+  // the sweep's multiply-adds (sweep_slice), so that U equals the fused merit pass's
+  double u[3], none[3];
+  gather_rows<double, G, false, false, 4>(a.W, a.wcol, off, total, rs, len, act, a.R, a.R, 0, 0, lds, u, none);
   if (act)
   {
     double R[3] = {a.R[4*(size_t)p], a.R[4*(size_t)p + 1], a.R[4*(size_t)p + 2]}, U[3];
@@ -381,7 +456,7 @@ __device__ __forceinline__ void merit_slice(const MeritArgs &a, int s, bool vali
 #pragma unroll
       for (int e = 0; e < 9; e ++) Wi[e] = a.Wd[(size_t)e*n + p];
       mv_add(Bv, Wi, R, U);
-      U[0] += u0; U[1] += u1; U[2] += u2;
+      U[0] += u[0]; U[1] += u[1]; U[2] += u[2];
       if (g == 0)
 #pragma unroll
         for (int k = 0; k < 3; k ++) a.U[(size_t)k*n + p] = U[k];
