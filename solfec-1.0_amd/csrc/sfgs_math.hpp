@@ -14,6 +14,7 @@
 // registers; there is no memory traffic here.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <climits>
 
 namespace sfgs {
 
@@ -254,107 +255,164 @@ __device__ __forceinline__ int de_saxce_feng(const RowLaw<T> &L, T eps, int maxi
   return iter;
 }
 
+// The local solve of a sweep launch is its longest chain: a wavefront issues one
+// instruction at a time, about five clocks each, so the loop costs its number of
+// instructions.  It is written for few of them (600 -> about 300 per FP64
+// iteration with sliding and sticking rows in one wavefront; 8.5-9.2k -> 6.5-7.0k
+// clocks for three iterations in FP64, 5.6k -> 4.7k in FP32; with selects for the
+// sliding entries instead of a branch 7.1k and 5.0k):
+//  * one system for all states, completed in a branch for sliding,
+//    instead of four branches whose nine entries meet in moves; one division
+//    serves sliding (1/|d_T|) and sticking (1/d_N);
+//  * the pivot exchanges only where a lane of the wavefront has one;
+//  * alfa, delta and beta only where a lane has R.d < 0 (alfa < 0 elsewhere
+//    leaves beta = 1);
+//  * the error bound by squares, |dR|^2 against eps^2 max(|R|^2, 1), with the
+//    quotient and the root only within their rounding of equality.
+// Every operation that reaches U, R or a decision is the one it was, with the
+// same rounding (the fused multiply-adds are explicit and contraction is off):
+// whether a row at rest counts as open hangs on the last bit of U_N.
+template <typename T> struct ErrBound {
+  T lo, hi;   // |dR|^2 / max(|R|^2, 1) surely at most eps^2, surely above it
+  __device__ __forceinline__ explicit ErrBound(T eps)
+  {
+    // the quotient and the root are within a few ulp: 1e-13 (FP64), 4e-6 (FP32)
+    const T e2 = eps*eps, m = sizeof(T) == 8 ? T(1e-13) : T(4e-6);
+    const bool ok = e2 > (sizeof(T) == 8 ? T(1e-290) : T(1e-30));
+    lo = ok ? e2*(T(1) - m) : T(-1);
+    hi = ok ? e2*(T(1) + m) : T(INFINITY);
+  }
+};
+
+// a 3x3 solve as solve3 (the same pivots and operations), in registers without
+// branches but the exchanges; singular is set instead of a return
+template <typename T>
+__device__ __forceinline__ void lu3(T a0, T a1, T a2, T a3, T a4, T a5, T a6, T a7, T a8, T b0, T b1, T b2, T &x0, T &x1,
+                                    T &x2, bool &singular)
+{
+#pragma clang fp contract(off)
+  T m = fabs(a0);
+  const bool p1 = fabs(a1) > m;
+  m = p1 ? fabs(a1) : m;
+  const bool p2 = fabs(a2) > m;
+  if (__any(p1 || p2))
+  {
+    // row 0 with row 2 where p2, else with row 1 where p1
+    const bool q1 = p1 && !p2;
+    T t;
+    t = a0; a0 = p2 ? a2 : q1 ? a1 : a0; a1 = q1 ? t : a1; a2 = p2 ? t : a2;
+    t = a3; a3 = p2 ? a5 : q1 ? a4 : a3; a4 = q1 ? t : a4; a5 = p2 ? t : a5;
+    t = a6; a6 = p2 ? a8 : q1 ? a7 : a6; a7 = q1 ? t : a7; a8 = p2 ? t : a8;
+    t = b0; b0 = p2 ? b2 : q1 ? b1 : b0; b1 = q1 ? t : b1; b2 = p2 ? t : b2;
+  }
+  const T i0 = fdiv(T(1), a0);
+  singular = a0 == T(0);
+  const T l1 = a1*i0, l2 = a2*i0;
+  a4 = fma(-l1, a3, a4); a7 = fma(-l1, a6, a7); b1 = fma(-l1, b0, b1);
+  a5 = fma(-l2, a3, a5); a8 = fma(-l2, a6, a8); b2 = fma(-l2, b0, b2);
+  const bool p = fabs(a5) > fabs(a4);
+  if (__any(p))
+  {
+    T t;
+    t = a4; a4 = p ? a5 : a4; a5 = p ? t : a5;
+    t = a7; a7 = p ? a8 : a7; a8 = p ? t : a8;
+    t = b1; b1 = p ? b2 : b1; b2 = p ? t : b2;
+  }
+  const T i1 = fdiv(T(1), a4);
+  singular = singular || a4 == T(0);
+  const T l = a5*i1;
+  a8 = fma(-l, a7, a8); b2 = fma(-l, b1, b2);
+  singular = singular || a8 == T(0);
+  x2 = b2*fdiv(T(1), a8);
+  x1 = fma(-x2, a7, b1)*i1;
+  x0 = fma(-x1, a3, fma(-x2, a6, b0))*i0;
+}
+
 template <typename T>
 __device__ __forceinline__ int semismooth_newton(const RowLaw<T> &L, T eps, int maxiter, const T *W, const T *B, T *U, T *R)
 {
+#pragma clang fp contract(off)
   if (L.separated) { R[0] = R[1] = R[2] = T(0); U[0] = B[0]; U[1] = B[1]; U[2] = B[2]; return 0; }
   const T fri = L.fri, coh = L.coh;
+  const ErrBound<T> bound(eps);
   T rho = L.rho;
-  int divi = maxiter / 10, iter = 0;
-  T err;
+  const int divi = maxiter / 10;
+  int iter = 0, left = divi > 0 ? divi : INT_MAX;
+  bool more;
   do
   {
-    T R0[3] = {R[0], R[1], R[2]}, RES[3], a[9], b[3], c[3], d[3];
-    T UN = U[2] + L.shift;
-    d[0] = R[0] - rho*U[0];
-    d[1] = R[1] - rho*U[1];
-    d[2] = (R[2] + coh) - rho*UN;
-    mv_add(B, W, R, RES);
-    RES[0] -= U[0]; RES[1] -= U[1]; RES[2] -= U[2];
-
-    if (d[2] >= T(0))
+    const T UN = U[2] + L.shift, RN = R[2] + coh;
+    const T d0 = fma(-rho, U[0], R[0]), d1 = fma(-rho, U[1], R[1]), d2 = fma(-rho, UN, RN);
+    const T s0 = (B[0] + fma(W[6], R[2], fma(W[3], R[1], W[0]*R[0]))) - U[0];
+    const T s1 = (B[1] + fma(W[7], R[2], fma(W[4], R[1], W[1]*R[0]))) - U[1];
+    const T s2 = (B[2] + fma(W[8], R[2], fma(W[5], R[1], W[2]*R[0]))) - U[2];
+    T x0 = -R[0], x1 = -R[1], x2 = -R[2];   // open: R = 0
+    if (d2 >= T(0))
     {
-      T norm = fsqrt(d[0]*d[0] + d[1]*d[1]);
-      T lim = fri * tmax(T(0), d[2]);
-      if (norm >= lim)
+      const T norm = fsqrt(fma(d0, d0, d1*d1)), lim = fri*d2;
+      const bool out = norm >= lim, slide = out && lim > T(0);
+      const T inv = fdiv(T(1), slide ? norm : d2);
+      const T s = fma(rho*U[2], inv, T(1));
+      T a0 = W[0], a1 = W[1], a3 = W[3], a4 = W[4], a6 = fma(U[0], inv, W[6]), a7 = fma(U[1], inv, W[7]);
+      T b0 = fma(-s, U[0], -s0), b1 = fma(-s, U[1], -s1);
+      const T b2 = -UN - s2;
+      if (out)
       {
-        if (lim > T(0))
+        if (slide)
         {
-          T len = fsqrt(R[0]*R[0] + R[1]*R[1]);
-          const T inorm = fdiv(T(1), norm);
-          T den = tmax(lim, len) * norm;
-          const T iden = fdiv(T(1), den);
-          T e = lim * inorm, beta;
-          if (len == T(0)) beta = T(1);
-          else
+          const T len = fsqrt(fma(R[1], R[1], R[0]*R[0])), r0 = R[0]*d0, r1 = R[1]*d1, num = r0 + r1;
+          const T iden = fdiv(T(1), tmax(lim, len)*norm), e = lim*inv;
+          T beta = T(1);
+          if (num < T(0) && len != T(0))
           {
-            T alfa = fdiv(R[0]*d[0] + R[1]*d[1], len*norm);
-            T delta = tmin(fdiv(len, lim), T(1));
-            beta = alfa < T(0) ? fdiv(T(1), T(1) - alfa*delta) : T(1);
+            const T alfa = fdiv(num, len*norm), delta = tmin(fdiv(len, lim), T(1));
+            beta = alfa < T(0) ? fdiv(T(1), fma(-alfa, delta, T(1))) : T(1);
           }
-          T F0 = (R[0]*d[0])*iden, F1 = (R[1]*d[0])*iden, F2 = (R[0]*d[1])*iden, F3 = (R[1]*d[1])*iden;
-          T M0 = e*(T(1) - F0), M1 = -e*F1, M2 = -e*F2, M3 = e*(T(1) - F3);
-          T H0 = T(1) - beta*M0, H1 = -beta*M1, H2 = -beta*M2, H3 = T(1) - beta*M3;
-          const T t0 = d[0]*inorm, t1 = d[1]*inorm;
-          a[0] = H0 + rho*(M0*W[0] + M2*W[1]);
-          a[1] = H1 + rho*(M1*W[0] + M3*W[1]);
-          a[2] = W[2];
-          a[3] = H2 + rho*(M0*W[3] + M2*W[4]);
-          a[4] = H3 + rho*(M1*W[3] + M3*W[4]);
-          a[5] = W[5];
-          a[6] = rho*(M0*W[6] + M2*W[7]) - fri*t0;
-          a[7] = rho*(M1*W[6] + M3*W[7]) - fri*t1;
-          a[8] = W[8];
-          b[0] = fri*t0*(R[2] + coh) - R[0] - rho*(M0*RES[0] + M2*RES[1]);
-          b[1] = fri*t1*(R[2] + coh) - R[1] - rho*(M1*RES[0] + M3*RES[1]);
-          b[2] = -UN - RES[2];
+          const T M0 = e*fma(-r0, iden, T(1)), M1 = -e*((R[1]*d0)*iden);
+          const T M2 = -e*((R[0]*d1)*iden), M3 = e*fma(-r1, iden, T(1));
+          const T f0 = fri*(d0*inv), f1 = fri*(d1*inv);
+          a0 = fma(rho, fma(W[1], M2, W[0]*M0), fma(-beta, M0, T(1)));
+          a1 = fma(rho, fma(W[0], M1, W[1]*M3), -(beta*M1));
+          a3 = fma(rho, fma(W[4], M2, W[3]*M0), -(beta*M2));
+          a4 = fma(rho, fma(W[3], M1, W[4]*M3), fma(-beta, M3, T(1)));
+          a6 = fma(rho, fma(W[7], M2, W[6]*M0), -f0);
+          a7 = fma(rho, fma(W[6], M1, W[7]*M3), -f1);
+          b0 = fma(-rho, fma(s1, M2, s0*M0), fma(RN, f0, -R[0]));
+          b1 = fma(-rho, fma(s0, M1, s1*M3), fma(RN, f1, -R[1]));
         }
         else
         {
-          a[0] = T(1); a[1] = T(0); a[2] = W[2];
-          a[3] = T(0); a[4] = T(1); a[5] = W[5];
-          a[6] = T(0); a[7] = T(0); a[8] = W[8];
-          b[0] = -R[0] - RES[0];
-          b[1] = -R[1] - RES[1];
-          b[2] = -UN - RES[2];
+          a0 = a4 = T(1);
+          a1 = a3 = a6 = a7 = T(0);
+          b0 = -R[0] - s0;
+          b1 = -R[1] - s1;
         }
       }
-      else
-      {
-#pragma unroll
-        for (int k = 0; k < 9; k ++) a[k] = W[k];
-        const T id2 = fdiv(T(1), d[2]);
-        a[6] += U[0]*id2;
-        a[7] += U[1]*id2;
-        T s = T(1) + rho*U[2]*id2;
-        b[0] = -s*U[0] - RES[0];
-        b[1] = -s*U[1] - RES[1];
-        b[2] = -UN - RES[2];
-      }
+      bool singular;
+      lu3(a0, a1, W[2], a3, a4, W[5], a6, a7, W[8], b0, b1, b2, x0, x1, x2, singular);
+      if (singular) return -1;
     }
-    else
-    {
-      a[0] = T(1); a[1] = T(0); a[2] = T(0);
-      a[3] = T(0); a[4] = T(1); a[5] = T(0);
-      a[6] = T(0); a[7] = T(0); a[8] = T(1);
-      b[0] = -R[0]; b[1] = -R[1]; b[2] = -R[2];
-    }
+    if (!isfinite(x0 + x1 + x2)) return -1;
 
-    if (solve3(a, b)) return -1;
-    if (!isfinite(b[0] + b[1] + b[2])) return -1;
-
-    mv_add(RES, W, b, c);
-    R[0] += b[0]; R[1] += b[1]; R[2] += b[2];
-    U[0] += c[0]; U[1] += c[1]; U[2] += c[2];
-    err = rel_change(R, R0);
+    U[0] += s0 + fma(W[6], x2, fma(W[3], x1, W[0]*x0));
+    U[1] += s1 + fma(W[7], x2, fma(W[4], x1, W[1]*x0));
+    U[2] += s2 + fma(W[8], x2, fma(W[5], x1, W[2]*x0));
+    const T p0 = R[0] + x0, p1 = R[1] + x1, p2 = R[2] + x2;
+    const T e0 = p0 - R[0], e1 = p1 - R[1], e2 = p2 - R[2];
+    R[0] = p0; R[1] = p1; R[2] = p2;
+    const T dd = fma(e2, e2, fma(e1, e1, e0*e0));
+    const T mx = tmax(fma(p2, p2, fma(p1, p1, p0*p0)), T(1));
+    more = dd > bound.hi*mx;
+    if (!more && !(dd < bound.lo*mx)) more = fsqrt(fdiv(dd, mx)) > eps;
     iter ++;
-    if (divi > 0 && iter % divi == 0)
+    if (-- left == 0)
     {
+      left = divi;
       rho *= T(10);
       if (isinf(rho)) return -1;
     }
   }
-  while (iter < maxiter && err > eps);
+  while (iter < maxiter && more);
   return iter;
 }
 
