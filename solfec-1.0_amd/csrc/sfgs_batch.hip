@@ -343,23 +343,23 @@ struct UScene {
   int slice0, slice1;     // the scene's slices (all colours)
 };
 
-// sbound: per slice, the rows already updated in this sweep (forward: the
-// scene's earlier colours; backward: its later ones)
+// list: per slice of the launch its number, its scene and the rows already updated
+// in this sweep (forward: the scene's earlier colours; backward: its later ones)
 template <typename T, int G, bool MERIT>
-__global__ __launch_bounds__(TPB) void k_usweep(SweepArgs<T> a, const int *clist, int nlist, const int2 *sbound,
-                                                const int *sscene, BatchOut *out, double *spart, int backward)
+__global__ __launch_bounds__(TPB) void k_usweep(SweepArgs<T> a, const int4 *list, int nlist, BatchOut *out,
+                                                double *spart, int backward)
 {
-  const int idx = blockIdx.x*(TPB/SLICE) + (threadIdx.x >> 6);
+  const int idx = __builtin_amdgcn_readfirstlane(blockIdx.x*(TPB/SLICE) + (threadIdx.x >> 6));
   if (idx >= nlist) return;                       // whole wavefront
-  const int s = clist[idx], sc = sscene[s];
-  BatchOut *o = out + sc;
-  if (o->done) return;                            // a finished scene: whole wavefront
-  const int2 bd = sbound[s];
+  const int4 e = list[idx];
+  const int s = e.x;
+  BatchOut *o = out + e.y;
   __shared__ T lds[TPB/SLICE][MERIT ? Gather<T>::LDS2 : Gather<T>::LDS1];
   double eu = 0.0, el = 0.0, up = 0.0;
   int sweepno = o->iters0 + o->sweeps;
-  sweep_slice<T, G, MERIT>(a, s, true, bd.x, bd.y, backward, &sweepno, &o->failkey, &o->failcount, &o->aborted,
-                           eu, el, up, lds[threadIdx.x >> 6]);
+  // a finished scene: whole wavefront
+  if (!sweep_slice<T, G, MERIT>(a, s, true, e.z, e.w, backward, &sweepno, &o->failkey, &o->failcount, &o->aborted,
+                                eu, el, up, lds[threadIdx.x >> 6], &o->done)) return;
   eu = wave_sum(eu); el = wave_sum(el); up = wave_sum(up);
   if ((threadIdx.x & 63) == 0)
   {
@@ -531,43 +531,41 @@ static int run_union(sfgs_ctx *ctx, const SFGS_PARAM *par, const BatchArgs<T> &b
   const bool mixed = par->precision == SFGS_PREC_MIXED;
   const int nomerit = par->meritval >= 1.0 ? 1 : 0, maxiter = par->maxiter;
   const int refine = mixed ? std::max(par->refine, 0) : 0;
-  // slices listed colour by colour (all scenes), their scene and the rows
-  // already updated when they run in a forward or a backward sweep
-  std::vector<int> clist, cstart((size_t)ncol + 1, 0), sscene((size_t)std::max(ns, 1), 0),
-                   sbound(4*(size_t)std::max(ns, 1), 0), uscene(2*(size_t)std::max(nsc, 1), 0);
-  for (int c = 0; c < ncol; c ++)
-  {
-    cstart[c] = (int)clist.size();
-    for (int q = 0; q < nsc; q ++)
+  // slices listed colour by colour (all scenes), with their scene and the rows
+  // already updated when they run in a forward (first half) or a backward sweep
+  std::vector<int> list, cstart((size_t)ncol + 1, 0), sscene((size_t)std::max(ns, 1), 0),
+                   uscene(2*(size_t)std::max(nsc, 1), 0);
+  list.reserve(8*(size_t)ns + 4);
+  for (int back = 0; back < 2; back ++)
+    for (int c = 0; c < ncol; c ++)
     {
-      const int g = q*ncol + c;
-      for (int sl = ctx->h_cslice[g]; sl < ctx->h_cslice[g + 1]; sl ++)
+      if (!back) cstart[c] = (int)(list.size()/4);
+      for (int q = 0; q < nsc; q ++)
       {
-        clist.push_back(sl);
-        sscene[sl] = q;
-        sbound[2*(size_t)sl] = ctx->h_colptr[(size_t)q*ncol];            // forward: the scene's earlier colours
-        sbound[2*(size_t)sl + 1] = ctx->h_colptr[g];
-        const size_t bb = 2*(size_t)std::max(ns, 1) + 2*(size_t)sl;      // backward: its later colours
-        sbound[bb] = ctx->h_colptr[g + 1];
-        sbound[bb + 1] = ctx->h_colptr[(size_t)(q + 1)*ncol];
+        const int g = q*ncol + c;
+        const int lo = back ? ctx->h_colptr[g + 1] : ctx->h_colptr[(size_t)q*ncol];
+        const int hi = back ? ctx->h_colptr[(size_t)(q + 1)*ncol] : ctx->h_colptr[g];
+        for (int sl = ctx->h_cslice[g]; sl < ctx->h_cslice[g + 1]; sl ++)
+        {
+          list.push_back(sl); list.push_back(q); list.push_back(lo); list.push_back(hi);
+          sscene[sl] = q;
+        }
       }
     }
-  }
-  cstart[ncol] = (int)clist.size();
+  cstart[ncol] = ns;
   for (int q = 0; q < nsc; q ++)
   {
     uscene[2*(size_t)q] = ctx->h_cslice[(size_t)q*ncol];
     uscene[2*(size_t)q + 1] = ctx->h_cslice[(size_t)(q + 1)*ncol];
   }
   const int maxsweeps = nomerit ? maxiter : maxiter + 1;
-  CHK(upload(ctx, ctx->u_clist, clist.data(), std::max(clist.size(), (size_t)1)));
+  CHK(upload(ctx, ctx->u_list, list.data(), list.size()));
   CHK(upload(ctx, ctx->u_sscene, sscene.data(), sscene.size()));
-  CHK(upload(ctx, ctx->u_sbound, sbound.data(), sbound.size()));
   CHK(upload(ctx, ctx->u_scene, uscene.data(), uscene.size()));
   CHK(ensure(ctx, ctx->u_spart, 3*(size_t)std::max(ns, 1)));
   CHK(ensure(ctx, ctx->u_active, (size_t)maxsweeps + 1));
   const UScene *usc = (const UScene*)ctx->u_scene.p;
-  const int2 *sbf = (const int2*)ctx->u_sbound.p, *sbb = sbf + std::max(ns, 1);
+  const int4 *listf = (const int4*)ctx->u_list.p, *listb = listf + ns;
   BatchOut *out = (BatchOut*)ctx->bout.p;
   double *spart = ctx->u_spart.p;
   const int sblk = (ns + TPB/SLICE - 1) / (TPB/SLICE);
@@ -603,11 +601,11 @@ static int run_union(sfgs_ctx *ctx, const SFGS_PARAM *par, const BatchArgs<T> &b
           if (nl == 0) continue;
           const dim3 grid((nl + TPB/SLICE - 1) / (TPB/SLICE));
           if (merit)
-            hipLaunchKernelGGL((k_usweep<TT, G, true>), grid, dim3(TPB), 0, st, a, ctx->u_clist.p + cstart[c], nl,
-                               back ? sbb : sbf, (const int*)ctx->u_sscene.p, out, spart, back);
+            hipLaunchKernelGGL((k_usweep<TT, G, true>), grid, dim3(TPB), 0, st, a,
+                               (back ? listb : listf) + cstart[c], nl, out, spart, back);
           else
-            hipLaunchKernelGGL((k_usweep<TT, G, false>), grid, dim3(TPB), 0, st, a, ctx->u_clist.p + cstart[c], nl,
-                               back ? sbb : sbf, (const int*)ctx->u_sscene.p, out, spart, back);
+            hipLaunchKernelGGL((k_usweep<TT, G, false>), grid, dim3(TPB), 0, st, a,
+                               (back ? listb : listf) + cstart[c], nl, out, spart, back);
         }
         hipLaunchKernelGGL(k_uscene, dim3(nsc), dim3(TPB), 0, st, 1, usc, (const double*)spart, out, bound, miniter,
                            nomerit, eps, meritval, kk, ctx->u_active.p);

@@ -33,7 +33,13 @@ struct Ctrl {
   double energy;    // free energy (merit denominator source)
 };
 
-struct RowData;  // forward
+// one slice of the sweep layout, read as one 32-byte scalar load
+struct alignas(32) SliceTab {
+  long long off;    // first block slot
+  int row0, nrows;  // its rows
+  int blocks;       // blocks of its rows
+  int pad[3];
+};
 
 } // namespace sfgs
 
@@ -79,6 +85,7 @@ struct sfgs_ctx {
   int nslices = 0;
   sfgs::DBuf<int> slice_row0, slice_nrows, slice_len;   // slice_len: blocks of the slice
   sfgs::DBuf<long long> slice_off;       // block offset of slice (in blocks, multiple of 64)
+  sfgs::DBuf<sfgs::SliceTab> slice_tab;  // the four together, for the sweeps
   long long sell_blocks = 0;             // total block slots, the last slot of each slice filled up
 
   // ---- permuted row data (colour-major order)
@@ -133,7 +140,7 @@ struct sfgs_ctx {
   sfgs::DBuf<double> bpart;
   sfgs::DBuf<unsigned char> bout;         // per-scene result records
   sfgs::DBuf<int> babort;
-  sfgs::DBuf<int> u_clist, u_sscene, u_sbound, u_scene, u_active;   // per-colour batch schedule
+  sfgs::DBuf<int> u_list, u_sscene, u_scene, u_active;   // per-colour batch schedule
   sfgs::DBuf<double> u_spart;
 
   // ---- device-resident time stepping (sfgs_dom.hip): body shapes and state

@@ -181,7 +181,7 @@ __global__ __launch_bounds__(64) void k_flow(FlowArgs<T> f)
       int ok = 1;
       {
         const int mine = total > lane ? (total - lane + SLICE - 1) / SLICE : 0;
-        const int *cb = a.wcol + a.off[s] + lane;
+        const int *cb = a.wcol + a.tab[s].off + lane;
         unsigned spins = 0;
         for (int m0 = 0; m0 < mine && ok; )
         {

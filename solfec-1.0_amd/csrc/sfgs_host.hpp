@@ -57,8 +57,8 @@ static SweepArgs<T> sweep_args(sfgs_ctx *ctx, const SFGS_PARAM *par, const T *W,
                                const T *rho, const T *fri, const T *coh, const T *shift, T *U, T *Um, double diageps)
 {
   SweepArgs<T> a;
-  a.row0 = ctx->slice_row0.p; a.nrows = ctx->slice_nrows.p; a.rowlen = ctx->rowlen.p; a.off = ctx->slice_off.p;
-  a.rowoff = ctx->rowoff.p; a.slen = ctx->slice_len.p;
+  a.row0 = ctx->slice_row0.p; a.nrows = ctx->slice_nrows.p; a.rowlen = ctx->rowlen.p;
+  a.rowoff = ctx->rowoff.p; a.slen = ctx->slice_len.p; a.tab = ctx->slice_tab.p;
   a.W = W; a.wcol = ctx->wcol.p; a.Wd = Wd; a.A = ctx->A.p; a.B = B; a.rho = rho;
   a.rec = sizeof(T) == 4 ? reinterpret_cast<const float4 *>(ctx->rec32.p) : nullptr;
   a.fri = fri; a.coh = coh; a.shift = shift; a.sep = ctx->sep.p;

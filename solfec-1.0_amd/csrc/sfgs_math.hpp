@@ -14,6 +14,7 @@
 // registers; there is no memory traffic here.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <cfloat>
 #include <climits>
 
 namespace sfgs {
@@ -31,6 +32,26 @@ template <typename T> __device__ __forceinline__ T fdiv(T a, T b) { return a / b
 template <> __device__ __forceinline__ float fdiv<float>(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
 template <typename T> __device__ __forceinline__ T fsqrt(T x) { return sqrt(x); }
 template <> __device__ __forceinline__ float fsqrt<float>(float x) { return __builtin_amdgcn_sqrtf(x); }
+
+// 1/x and 1/sqrt(x) in FP64 for normal x (rsqrt64: positive), from the hardware
+// estimates by Newton's iteration, to about one ulp: the estimates are good to
+// 2^-22 or better, so two steps reach 2^-53.  The caller excludes zero,
+// subnormal and infinite arguments.
+__device__ __forceinline__ double rcp64(double x)
+{
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(r, fma(-x, r, 1.0), r);
+  return fma(r, fma(-x, r, 1.0), r);
+}
+__device__ __forceinline__ double rsqrt64(double x)
+{
+  const double y = __builtin_amdgcn_rsq(x);
+  double h = 0.5*y, g = x*y, e = fma(-h, g, 0.5);
+  h = fma(h, e, h); g = fma(g, e, g);
+  e = fma(-h, g, 0.5);
+  h = fma(h, e, h);
+  return h + h;
+}
 
 // y = c + M v
 template <typename T>
@@ -197,6 +218,29 @@ __device__ __forceinline__ void scf_residual(T fri, T coh, T shift, const T *U, 
       for (int r = 0; r < 3; r ++)
         X[r + 3*c] = dF[r + 3*c] - (Y[r]*dF[3*c] + Y[r + 3]*dF[3*c + 1] + Y[r + 6]*dF[3*c + 2]);
   }
+}
+
+// C(U,R) of the merit in FP64: scf_residual without the Jacobians, with the
+// quotients shared (1/(1 + mu^2) once, |U_T| and 1/|S_T| from one reciprocal root
+// each) instead of three roots and five divisions, which took 920 of a slice's
+// clocks.  A tangential part whose square is subnormal counts as none: u2 = (1, 0)
+// as in spectral.  Only the merit sums depend on it.
+__device__ __forceinline__ void merit_residual(double fri, double coh, double shift, const double *U, const double *R,
+                                               double *C)
+{
+  const double io = rcp64(1.0 + fri*fri);
+  const double uu = U[0]*U[0] + U[1]*U[1];
+  const double ulen = uu >= DBL_MIN ? uu*rsqrt64(uu) : 0.0;
+  const double F2 = U[2] + shift + fri*ulen;
+  const double S0 = R[0] - U[0], S1 = R[1] - U[1], S2 = R[2] - F2 + coh;
+  const double ss = S0*S0 + S1*S1;
+  const bool on = ss >= DBL_MIN;
+  const double is = on ? rsqrt64(ss) : 0.0, sl = ss*is;
+  const double g1 = fmax(-(S2 + fri*sl), 0.0)*io, g2 = fmax(sl - fri*S2, 0.0)*io;
+  const double gt = g2 - fri*g1;
+  C[0] = U[0] + gt*(on ? S0*is : 1.0);
+  C[1] = U[1] + gt*(S1*is);
+  C[2] = F2 - (g1 + fri*g2);
 }
 
 // per-row constants of the local problem

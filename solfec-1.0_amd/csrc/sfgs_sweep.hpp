@@ -39,10 +39,10 @@ __device__ __forceinline__ T wave_sum(T v)
 
 template <typename T>
 struct SweepArgs {
-  const int *row0, *nrows, *rowlen;
+  const int *row0, *nrows, *rowlen;   // row0, nrows, slen: as in tab
   const int *rowoff;    // first block of each row in its slice
-  const int *slen;      // blocks of each slice
-  const long long *off;
+  const int *slen;
+  const SliceTab *tab;
   const T *W;
   const int *wcol;
   const T *Wd, *B, *rho, *fri, *coh, *shift;
@@ -256,27 +256,34 @@ __device__ __forceinline__ void gather_rows(const T *W, const int *wcol, long lo
   for (int c = 0; c < 3; c ++) { b[c] = gsum<G>(b[c]); if (TWO) u[c] = gsum<G>(u[c]); }
 }
 
-// One slice (64/G rows of one colour, one wavefront) of a sweep.  eu, el and
+// One slice (64/G rows of one colour, one wavefront) of a sweep; false when *stop
+// (a solve that has stopped; null: none) left it untouched.  eu, el and
 // up receive this lane's contributions to the error sums and to the merit
 // numerator.  A failed local solve is recorded in failkey / failcount, keyed by
-// the sweep number *sweepno, and raises *abortflag under FAILURE_EXIT.  run =
-// false (a solve that has stopped) leaves the slice untouched; the caller reads
-// that flag together with the slice table, so both cost one memory round trip.
+// the sweep number *sweepno, and raises *abortflag under FAILURE_EXIT.  The flag
+// is read together with the slice table, so both cost one memory round trip.
 // COH: P and Q are shared with other wavefronts of the same launch (r_ld / r_st).
 // lds: this wavefront's Gather<T>::LDS2 (merit) or LDS1 values.  s and valid are
 // the same in all lanes of the wavefront.
 template <typename T, int G, bool MERIT, bool COH = false>
-__device__ __forceinline__ void sweep_slice(const SweepArgs<T> &a, int s, bool valid, int upd_lo, int upd_hi,
+__device__ __forceinline__ bool sweep_slice(const SweepArgs<T> &a, int s, bool valid, int upd_lo, int upd_hi,
                                             int backward, const int *sweepno, unsigned long long *failkey,
                                             int *failcount, int *abortflag, double &eu, double &el, double &up,
-                                            T *lds, bool run = true)
+                                            T *lds, const int *stop = nullptr)
 {
   const int l = threadIdx.x & 63, r = l / G, g = l % G;
   const int n = a.n;
+  if (!__builtin_amdgcn_readfirstlane(valid)) return !(stop && *stop);
   s = __builtin_amdgcn_readfirstlane(s);
-  if (!__builtin_amdgcn_readfirstlane(valid && run)) return;
-  const int nr = a.nrows[s], r0 = a.row0[s], total = a.slen[s];   // one round of loads
-  const long long off = a.off[s];
+  const SliceTab tab = a.tab[s];
+  const int stopped = __builtin_amdgcn_readfirstlane(stop ? *stop : 0);
+  const int nr = __builtin_amdgcn_readfirstlane(tab.nrows), r0 = __builtin_amdgcn_readfirstlane(tab.row0);
+  const int total = __builtin_amdgcn_readfirstlane(tab.blocks);
+  const long long off = (long long)__builtin_amdgcn_readfirstlane((int)(tab.off >> 32)) << 32 |
+                        (unsigned)__builtin_amdgcn_readfirstlane((int)tab.off);
+  // all of them loaded here, none behind the branch
+  asm volatile("" :: "s"(nr), "s"(r0), "s"(total), "s"(off), "s"(stopped));
+  if (stopped) return false;
   const bool act = r < nr;
   // The row's own data first, so that its loads are in flight with the gather's.
   // Nothing is computed from them before the gather (a use waits for them), and
@@ -348,7 +355,7 @@ __device__ __forceinline__ void sweep_slice(const SweepArgs<T> &a, int s, bool v
       U[0] += u[0]; U[1] += u[1]; U[2] += u[2];
       // the merit is evaluated in FP64 whatever the sweep type
       double C[3], Ud[3] = {U[0], U[1], U[2]}, Rd[3] = {R[0], R[1], R[2]};
-      scf_residual<double>(L.fri, L.coh, L.shift, Ud, Rd, C, nullptr, nullptr);
+      merit_residual(L.fri, L.coh, L.shift, Ud, Rd, C);
       const double q0 = Ai[0]*C[0] + Ai[3]*C[1] + Ai[6]*C[2];
       const double q1 = Ai[1]*C[0] + Ai[4]*C[1] + Ai[7]*C[2];
       const double q2 = Ai[2]*C[0] + Ai[5]*C[1] + Ai[8]*C[2];
@@ -408,6 +415,7 @@ __device__ __forceinline__ void sweep_slice(const SweepArgs<T> &a, int s, bool v
       el += (double)R[0]*R[0] + (double)R[1]*R[1] + (double)R[2]*R[2];
     }
   }
+  return true;
 }
 
 // standalone merit (MERIT_Function with update_U, mrf.c:35-184) on the
@@ -467,7 +475,7 @@ __device__ __forceinline__ void merit_slice(const MeritArgs &a, int s, bool vali
       for (int k = 0; k < 3; k ++) U[k] = a.U[(size_t)k*n + p];
     }
     double C[3], Ai[9];
-    scf_residual<double>(a.fri[p], a.coh[p], a.shift[p], U, R, C, nullptr, nullptr);
+    merit_residual(a.fri[p], a.coh[p], a.shift[p], U, R, C);
 #pragma unroll
     for (int e = 0; e < 9; e ++) Ai[e] = a.A[(size_t)e*n + p];
     const double q0 = Ai[0]*C[0] + Ai[3]*C[1] + Ai[6]*C[2];
