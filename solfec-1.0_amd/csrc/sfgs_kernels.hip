@@ -1252,10 +1252,29 @@ static int colour_graph(sfgs_ctx *ctx, int n)
   return 0;
 }
 
-// permutation into colour-major order and the SELL-64 slice table
+// Rows of a slice for a colour of n rows (all scenes): 64/G, what the lanes of a
+// wavefront hold, or half of that in a colour that then has at most HALF_SLICES
+// slices and is past the group launch.  Such a colour leaves SIMDs idle and its
+// launch takes as long as one wavefront: with half the rows that one gathers half
+// the slots of blocks and runs fewer Newton iterations (the most any of its rows
+// needs).  Measured in us a sweep, 64/G rows against this: 7919 rows 100.0 and
+// 93.2, 60001 ellipsoids 104.4 and 101.9, 200k 206.4 and 201.6, 200k mixed 111.2
+// and 108.5; 1000 and 1331 rows the same.  Quarters or eighths add nothing there
+// and cost where colours are small (1331 rows 61.8, 63.8 and 69.7; 1000 rows 74.4,
+// 76.2 and 76.4: more partial sums to add up at the end), and so do halves in the
+// group launch (216 rows 46.3 and 51.6).  1024 in place of 512: 200k 203.4, 60001
+// 103.3.  The iterates do not depend on it.
+static const int GROUP_NW = 8, HALF_SLICES = 512;
+static int slice_rows(int n, int G)
+{
+  const int full = SLICE / G, half = full / 2;
+  return n > GROUP_NW*full && n <= HALF_SLICES*half ? half : full;
+}
+
+// permutation into colour-major order and the slice table
 static int build_order(sfgs_ctx *ctx, int n, bool have_master)
 {
-  const int G = ctx->G, RPS = SLICE / G;
+  const int G = ctx->G;
   const bool scenes = ctx->nscenes > 1;
   ctx->G_built = G;
   CHK(ensure(ctx, ctx->skeys, n));
@@ -1314,14 +1333,17 @@ static int build_order(sfgs_ctx *ctx, int n, bool have_master)
   HIPCHK(hipStreamSynchronize(ctx->stream));
   ctx->h_colptr.assign((size_t)nc + 1, 0);
   ctx->h_cslice.assign((size_t)nc + 1, 0);
-  std::vector<int> row0, nrows;
+  std::vector<int> row0, nrows, rps((size_t)std::max(ncol, 1), 0);
+  for (int c = 0; c < nc; c ++) rps[c % ncol] += cnt[c];
+  for (int &r : rps) r = slice_rows(r, G);
   for (int c = 0; c < nc; c ++)
   {
     ctx->h_colptr[c + 1] = ctx->h_colptr[c] + cnt[c];
-    for (int r = ctx->h_colptr[c]; r < ctx->h_colptr[c + 1]; r += RPS)
+    const int m = rps[c % ncol];
+    for (int r = ctx->h_colptr[c]; r < ctx->h_colptr[c + 1]; r += m)
     {
       row0.push_back(r);
-      nrows.push_back(std::min(RPS, ctx->h_colptr[c + 1] - r));
+      nrows.push_back(std::min(m, ctx->h_colptr[c + 1] - r));
     }
     ctx->h_cslice[c + 1] = (int)row0.size();
   }
@@ -1784,11 +1806,9 @@ int SFGS_System_Upload(sfgs_ctx *ctx, int n, const int *rowptr, const int *col, 
   case 8: SFGS_SWEEP_WPB(MER, 8) break; \
   default: SFGS_SWEEP_WPB(MER, 4) break; }
 
-// the trailing colours merged into one k_sweep_group launch: wavefronts of its
-// workgroup, and the most slices a colour may have to join it (one slice per
-// wavefront)
-static const int GROUP_NW = 8;
-
+// the trailing colours merged into one k_sweep_group launch: GROUP_NW wavefronts
+// in its workgroup, and the most slices a colour may have to join it (one slice
+// per wavefront)
 #define SFGS_GROUP_LAUNCH(MER, GG) \
   hipLaunchKernelGGL((k_sweep_group<T, GG, MER, GROUP_NW>), dim3(1), dim3(GROUP_NW*64), 0, ctx->stream, a, cg, \
                      gslot, backward, f, np, hist);
