@@ -1257,14 +1257,21 @@ static int colour_graph(sfgs_ctx *ctx, int n)
 // slices and is past the group launch.  Such a colour leaves SIMDs idle and its
 // launch takes as long as one wavefront: with half the rows that one gathers half
 // the slots of blocks and runs fewer Newton iterations (the most any of its rows
-// needs).  Measured in us a sweep, 64/G rows against this: 7919 rows 100.0 and
+// needs).
+// GROUP_NW: the wavefronts of the group launch and the most slices of a colour in it.
+// One CU's misses are what bounds that launch (the gather of a slice takes 3-4k
+// cycles alone and 18-21k beside six others there), so only colours with one slice
+// per SIMD of the CU are worth the launch they save; 8, 4, 3, 2 slices measured in
+// us a sweep: 216 rows 44.9, 43.9, 47.0, 51.4; 1000 rows 74.4, 71.9, 72.4, 73.2; 7919
+// rows 93.4, 88.0, 87.7, 87.6; 200k 200.6, 193.4, 192.5, 193.3.
+// Halves, in us a sweep (with a group of 8), 64/G rows against this: 7919 rows 100.0 and
 // 93.2, 60001 ellipsoids 104.4 and 101.9, 200k 206.4 and 201.6, 200k mixed 111.2
 // and 108.5; 1000 and 1331 rows the same.  Quarters or eighths add nothing there
 // and cost where colours are small (1331 rows 61.8, 63.8 and 69.7; 1000 rows 74.4,
 // 76.2 and 76.4: more partial sums to add up at the end), and so do halves in the
 // group launch (216 rows 46.3 and 51.6).  1024 in place of 512: 200k 203.4, 60001
 // 103.3.  The iterates do not depend on it.
-static const int GROUP_NW = 8, HALF_SLICES = 512;
+static const int GROUP_NW = 4, HALF_SLICES = 512;
 static int slice_rows(int n, int G)
 {
   const int full = SLICE / G, half = full / 2;
