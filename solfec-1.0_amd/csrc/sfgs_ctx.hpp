@@ -85,6 +85,7 @@ struct sfgs_ctx {
   int nslices = 0;
   sfgs::DBuf<int> slice_row0, slice_nrows, slice_len;   // slice_len: blocks of the slice
   sfgs::DBuf<long long> slice_off;       // block offset of slice (in blocks, multiple of 64)
+  sfgs::DBuf<long long> slice_lens;      // build_order: block slots of every slice, for the offsets
   sfgs::DBuf<sfgs::SliceTab> slice_tab;  // the four together, for the sweeps
   long long sell_blocks = 0;             // total block slots, the last slot of each slice filled up
 

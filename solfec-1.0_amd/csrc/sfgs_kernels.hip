@@ -227,6 +227,95 @@ __global__ void k_jp_round(int n, const int *rowptr, const int *col, const int *
   atomicMax(maxcol, c);
 }
 
+// The same colouring of a symmetric graph in place: there a vertex is coloured
+// after all neighbours that outrank it and before all others, so the colours are
+// greedy first-fit whenever each one is written, and no second buffer, copy or
+// round of all vertices is needed.  (An uploaded structure may be unsymmetric; its
+// colours are those of the rounds above.)  A thread takes its neighbours eight at
+// a time, all loads in flight, and looks again at those that outrank it and are
+// uncoloured; colours go through device-scope accesses, so a vertex is seen in a
+// microsecond wherever it was coloured, and a chain of dependent vertices costs
+// that and not a launch with a host round trip each.  It waits for nobody: after
+// JP_LOOKS looks without having finished it leaves the vertex to the next launch,
+// which *before (the vertices that this launch's predecessor left) may end at once.
+// Bound by the looks: 417k vertices of 7.4 neighbours in 0.69 ms (573 + 96 + 12 + 6 us
+// the four launches) against 34 rounds of 96 us, 690 vertices in 70 us against 0.7 ms;
+// the assembly as a whole 5.45 -> 2.07 ms and 0.97 -> 0.36 ms.
+static const int JP_LOOKS = 64, JP_LAUNCHES = 4;
+
+__global__ __launch_bounds__(TPB) void k_jp_inplace(int n, const int *rowptr, const int *col, int *colour,
+                                                    const int *before, int *remaining, int *maxcol)
+{
+  if (before && *before == 0) return;
+  constexpr int CH = 8, NM = SFGS_MAX_COLOURS/64;
+  const int v = blockIdx.x*blockDim.x + threadIdx.x;
+  bool todo = v < n && colour[v] < 0;
+  int p = 0, end = 0, cmax = -1;
+  if (todo) { p = rowptr[v]; end = rowptr[v + 1]; }
+  const unsigned dv = (unsigned)(end - p), hv = hash32((unsigned)v);
+  unsigned long long mask[NM] = {0ull, 0ull, 0ull, 0ull};
+  int u[CH];
+  unsigned wait = 0;          // of u: outrank v and have shown no colour yet
+  bool loaded = false;
+  for (int look = 0; look < JP_LOOKS && __any(todo); look ++)
+  {
+    if (!todo) continue;
+    while (true)
+    {
+      if (!loaded && p < end)
+      {
+        unsigned d[CH];
+#pragma unroll
+        for (int q = 0; q < CH; q ++) u[q] = col[min(p + q, end - 1)];
+#pragma unroll
+        for (int q = 0; q < CH; q ++) d[q] = (unsigned)(rowptr[u[q] + 1] - rowptr[u[q]]);
+        wait = 0;
+#pragma unroll
+        for (int q = 0; q < CH; q ++)
+        {
+          const unsigned hu = hash32((unsigned)u[q]);
+          const bool above = d[q] != dv ? d[q] > dv : hu != hv ? hu > hv : u[q] > v;
+          if (above && p + q < end) wait |= 1u << q;
+        }
+        loaded = true;
+      }
+      int c[CH];
+#pragma unroll
+      for (int q = 0; q < CH; q ++)
+        c[q] = (wait >> q) & 1u ? __hip_atomic_load(colour + u[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : -1;
+#pragma unroll
+      for (int q = 0; q < CH; q ++)
+        if (c[q] >= 0)
+        {
+          wait &= ~(1u << q);
+#pragma unroll
+          for (int w = 0; w < NM; w ++) if (c[q] >> 6 == w) mask[w] |= 1ull << (c[q] & 63);
+        }
+      if (wait) break;
+      p += CH;
+      loaded = false;
+      if (p >= end) break;
+    }
+    if (!wait)
+    {
+      int c = SFGS_MAX_COLOURS;
+#pragma unroll
+      for (int w = NM - 1; w >= 0; w --) if (~mask[w]) c = 64*w + __ffsll((long long)~mask[w]) - 1;
+      __hip_atomic_store(colour + v, c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      cmax = c;
+      todo = false;
+    }
+  }
+  const int left = __popcll(__ballot(todo));
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) cmax = max(cmax, __shfl_xor(cmax, o, 64));
+  if ((threadIdx.x & 63) == 0)
+  {
+    if (left) atomicAdd(remaining, left);
+    if (cmax > __hip_atomic_load(maxcol, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(maxcol, cmax);
+  }
+}
+
 __global__ void k_copy_int(int n, const int *a, int *b)
 {
   int i = blockIdx.x*blockDim.x + threadIdx.x;
@@ -1224,12 +1313,37 @@ static int scan_ll(sfgs_ctx *ctx, const long long *in, long long *out, int n)
   return 0;
 }
 
-// colour the natural CSR (ctx->rowptr/col, n rows) into ctx->colour; sets ncolours
-static int colour_graph(sfgs_ctx *ctx, int n)
+// colour the natural CSR (ctx->rowptr/col, n rows) into ctx->colour; sets ncolours.
+// symmetric: the structure is known to be (an assembled one)
+static int colour_graph(sfgs_ctx *ctx, int n, bool symmetric)
 {
   ctx->ncolours = 0;
   if (n == 0) return 0;
   CHK(ensure(ctx, ctx->colour, n));
+  if (symmetric)
+  {
+    // counter: vertices left by each of JP_LAUNCHES launches, the largest colour
+    CHK(ensure(ctx, ctx->counter, JP_LAUNCHES + 1));
+    int *cnt = ctx->counter.p, h[JP_LAUNCHES + 1];
+    hipLaunchKernelGGL(k_fill_int, dim3(nblk(n)), dim3(TPB), 0, ctx->stream, n, -1, ctx->colour.p);
+    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(TPB), 0, ctx->stream, JP_LAUNCHES + 1, 0, cnt);
+    for (int round = 0; ; round ++)
+    {
+      // every launch with vertices left colours at least the one that outranks the others
+      if (round > n) { ctx->err = "colouring did not finish"; return SFGS_E_STATE; }
+      if (round > 0) hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(TPB), 0, ctx->stream, JP_LAUNCHES, 0, cnt);
+      for (int q = 0; q < JP_LAUNCHES; q ++)
+        hipLaunchKernelGGL(k_jp_inplace, dim3(nblk(n)), dim3(TPB), 0, ctx->stream, n, ctx->rowptr.p, ctx->col.p,
+                           ctx->colour.p, q > 0 ? cnt + q - 1 : (const int *)nullptr, cnt + q, cnt + JP_LAUNCHES);
+      HIPCHK(hipMemcpyAsync(h, cnt, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
+      HIPCHK(hipStreamSynchronize(ctx->stream));
+      HIPCHK(hipGetLastError());
+      if (h[JP_LAUNCHES - 1] == 0) break;
+    }
+    if (h[JP_LAUNCHES] >= SFGS_MAX_COLOURS) { ctx->err = "contact graph needs more than 256 colours"; return SFGS_E_COLOURS; }
+    ctx->ncolours = h[JP_LAUNCHES] + 1;
+    return 0;
+  }
   CHK(ensure(ctx, ctx->colour2, n));
   CHK(ensure(ctx, ctx->counter, 4));
   hipLaunchKernelGGL(k_fill_int, dim3(nblk(n)), dim3(TPB), 0, ctx->stream, n, -1, ctx->colour.p);
@@ -1359,9 +1473,8 @@ static int build_order(sfgs_ctx *ctx, int n, bool have_master)
   CHK(upload(ctx, ctx->slice_row0, row0.data(), (size_t)ns));
   CHK(upload(ctx, ctx->slice_nrows, nrows.data(), (size_t)ns));
   CHK(ensure(ctx, ctx->slice_len, (size_t)ns + 1));
-  DBuf<long long> &tmp = ctx->slice_off;  // reuse: lengths first, then offsets
-  CHK(ensure(ctx, tmp, (size_t)ns + 1));
-  DBuf<long long> lens;
+  CHK(ensure(ctx, ctx->slice_off, (size_t)ns + 1));
+  DBuf<long long> &lens = ctx->slice_lens;
   CHK(ensure(ctx, lens, (size_t)ns + 1));
   HIPCHK(hipMemsetAsync(lens.p, 0, sizeof(long long)*((size_t)ns + 1), ctx->stream));
   if (ns > 0)
@@ -1375,7 +1488,6 @@ static int build_order(sfgs_ctx *ctx, int n, bool have_master)
   long long total = 0;
   HIPCHK(hipMemcpyAsync(&total, ctx->slice_off.p + ns, sizeof(long long), hipMemcpyDeviceToHost, ctx->stream));
   HIPCHK(hipStreamSynchronize(ctx->stream));
-  release(lens);
   ctx->sell_blocks = total;
   CHK(ensure(ctx, ctx->W, (size_t)(9*total)));
   CHK(ensure(ctx, ctx->wcol, (size_t)total));
@@ -1542,7 +1654,7 @@ void SFGS_Destroy(sfgs_ctx *ctx)
   release(ctx->rowptr); release(ctx->rowlen_n); release(ctx->col); release(ctx->via);
   release(ctx->colour); release(ctx->colour2); release(ctx->perm); release(ctx->iperm); release(ctx->counter);
   release(ctx->skeys); release(ctx->skeys2); release(ctx->svals); release(ctx->svals2); release(ctx->scratch); release(ctx->bbox);
-  release(ctx->slice_row0); release(ctx->slice_nrows); release(ctx->slice_len); release(ctx->slice_off); release(ctx->slice_tab);
+  release(ctx->slice_row0); release(ctx->slice_nrows); release(ctx->slice_len); release(ctx->slice_off); release(ctx->slice_lens); release(ctx->slice_tab);
   release(ctx->rowlen); release(ctx->rowoff); release(ctx->W); release(ctx->Wd); release(ctx->A); release(ctx->B); release(ctx->V);
   release(ctx->rho); release(ctx->pfri); release(ctx->pcoh); release(ctx->shift); release(ctx->R); release(ctx->U); release(ctx->pen); sfgs_newton_release(ctx); sfgs_bar_release(ctx);
   release(ctx->Rb); release(ctx->Um); release(ctx->sep); release(ctx->wcol);
@@ -1681,7 +1793,7 @@ static int locdyn_update(sfgs_ctx *ctx, double step, int dynamic, bool full)
                        ctx->bptr.p, ctx->blist.p, ctx->rowptr.p, ctx->col.p, ctx->via.p);
 
   // colouring and colour-major layout
-  CHK(colour_graph(ctx, nc));
+  CHK(colour_graph(ctx, nc, true));
   CHK(build_order(ctx, nc, true));
   CHK(ensure_rows(ctx, nc));
 
@@ -1762,7 +1874,7 @@ int SFGS_System_Upload(sfgs_ctx *ctx, int n, const int *rowptr, const int *col, 
   CHK(upload(ctx, dgap, gap, (size_t)n));
   CHK(upload(ctx, ctx->Rn, R, 3*(size_t)n));
   CHK(upload(ctx, ctx->Un, U, 3*(size_t)n));
-  int rc = colour_graph(ctx, n);
+  int rc = colour_graph(ctx, n, false);
   if (!rc) rc = build_order(ctx, n, false);
   if (!rc) rc = ensure_rows(ctx, n);
   if (!rc && n > 0)
@@ -2536,7 +2648,7 @@ int SFGS_Colour(sfgs_ctx *ctx, int n, const int *rowptr, const int *col, int *co
   CHK(upload(ctx, ctx->rowptr, rowptr, (size_t)n + 1));
   CHK(upload(ctx, ctx->col, col, (size_t)nnz));
   ctx->assembled = 0;
-  CHK(colour_graph(ctx, n));
+  CHK(colour_graph(ctx, n, false));
   if (n > 0) HIPCHK(hipMemcpyAsync(colour, ctx->colour.p, sizeof(int)*(size_t)n, hipMemcpyDeviceToHost, ctx->stream));
   HIPCHK(hipStreamSynchronize(ctx->stream));
   return ctx->ncolours;
