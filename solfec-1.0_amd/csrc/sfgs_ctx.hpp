@@ -116,6 +116,7 @@ struct sfgs_ctx {
   int upmin = 0;                         // diagonal blocks only (SFGS_Locdyn_Update_Min): W products through the bodies
   sfgs::DBuf<double> pen;                // penalty solve: spring, dashpot, hpow per contact, or the default six
   sfgs::DBuf<double> nt_mem;             // Newton solve: linearisation, Krylov vectors, partials
+  sfgs::DBuf<unsigned char> nt_ctl;      // its control block (diagonal systems)
   sfgs::DBuf<unsigned char> bar_mem;     // barrier schedule: colour tables, partials, counter
 
   // ---- reductions / control

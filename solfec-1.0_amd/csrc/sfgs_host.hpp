@@ -72,13 +72,16 @@ static SweepArgs<T> sweep_args(sfgs_ctx *ctx, const SFGS_PARAM *par, const T *W,
 [[maybe_unused]] static MeritArgs merit_args(sfgs_ctx *ctx, int update_U, double *conmerit)
 {
   MeritArgs m;
-  m.row0 = ctx->slice_row0.p; m.nrows = ctx->slice_nrows.p; m.rowlen = ctx->rowlen.p; m.off = ctx->slice_off.p;
-  m.rowoff = ctx->rowoff.p; m.slen = ctx->slice_len.p;
+  m.tab = ctx->slice_tab.p; m.rowlen = ctx->rowlen.p; m.rowoff = ctx->rowoff.p;
   m.W = ctx->W.p; m.wcol = ctx->wcol.p; m.Wd = ctx->Wd.p; m.A = ctx->A.p; m.B = ctx->B.p; m.fri = ctx->pfri.p;
   m.coh = ctx->pcoh.p; m.shift = ctx->shift.p; m.R = ctx->R.p; m.U = ctx->U.p; m.n = ctx->nc; m.update_U = update_U;
-  m.mpartials = ctx->mpartials.p; m.conmerit = conmerit;
+  m.mpartials = ctx->mpartials.p; m.conmerit = conmerit; m.stop = nullptr;
   return m;
 }
+
+// k_merit over all slices on the context's stream, its mgrid partial sums in
+// ctx->mpartials; stop: as MeritArgs
+int launch_merit(sfgs_ctx *ctx, int update_U, double *conmerit, const int *stop, int *mgrid);
 
 // the sweeps of SFGS_Solve as one persistent dataflow launch (sfgs_flow.hip);
 // the final R and U are left in X0 and sa.U, hc.final_buf = hc.final_U = 0

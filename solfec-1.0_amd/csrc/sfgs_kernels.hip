@@ -818,6 +818,7 @@ __global__ __launch_bounds__(TPB) void k_merit(MeritArgs a, int nslices)
   __shared__ double lds[TPB/SLICE][Gather<double>::LDS1];
   double up = 0.0, z1 = 0.0, z2 = 0.0;
   merit_slice<G>(a, s, s < nslices, up, lds[threadIdx.x >> 6]);
+  if (a.stop && *a.stop) return;
   block_sum3(up, z1, z2);
   if (threadIdx.x == 0) a.mpartials[blockIdx.x] = up;
 }
@@ -2097,6 +2098,22 @@ int sfgs::build_f32_mirror(sfgs_ctx *ctx)
   return 0;
 }
 
+int sfgs::launch_merit(sfgs_ctx *ctx, int update_U, double *conmerit, const int *stop, int *mgrid)
+{
+  const int grid = (ctx->nslices + TPB/SLICE - 1) / (TPB/SLICE);
+  CHK(ensure(ctx, ctx->mpartials, (size_t)std::max(grid, 1)));
+  MeritArgs ma = merit_args(ctx, update_U, conmerit);
+  ma.stop = stop;
+  if (grid > 0)
+  {
+    SFGS_DISPATCH_G(ctx->G_built, auto kern = k_merit<GG>; hipLaunchKernelGGL(kern, dim3(grid), dim3(TPB), 0, ctx->stream,
+                    ma, ctx->nslices));
+  }
+  HIPCHK(hipGetLastError());
+  *mgrid = grid;
+  return 0;
+}
+
 extern "C" {
 
 int SFGS_Solve(sfgs_ctx *ctx, const SFGS_PARAM *par, double *rerhist, double *merhist, SFGS_REPORT *rep)
@@ -2363,12 +2380,11 @@ int SFGS_Merit(sfgs_ctx *ctx, int update_U, double *merit, double *conmerit)
   }
   HIPCHK(hipSetDevice(ctx->device));
   hipStream_t st = ctx->stream;
-  const int n = ctx->nc, mgrid = (ctx->nslices + TPB/SLICE - 1) / (TPB/SLICE);
-  CHK(ensure(ctx, ctx->mpartials, (size_t)std::max(mgrid, 1)));
+  const int n = ctx->nc;
+  int mgrid = 0;
   DBuf<double> cm;
   if (conmerit) { CHK(ensure(ctx, cm, (size_t)n)); }
-  MeritArgs ma = merit_args(ctx, update_U, conmerit ? cm.p : nullptr);
-  if (mgrid > 0) { SFGS_DISPATCH_G(ctx->G_built, auto kern = k_merit<GG>; hipLaunchKernelGGL(kern, dim3(mgrid), dim3(TPB), 0, st, ma, ctx->nslices)); }
+  CHK(sfgs::launch_merit(ctx, update_U, conmerit ? cm.p : nullptr, nullptr, &mgrid));
   std::vector<double> mp((size_t)std::max(mgrid, 1), 0.0);
   std::vector<double> hcm(conmerit ? (size_t)n : 0);
   std::vector<int> hperm(conmerit ? (size_t)n : 0);

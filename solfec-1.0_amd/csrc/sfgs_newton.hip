@@ -57,9 +57,62 @@ struct NtRows {
   int *singular;
 };
 
-__global__ __launch_bounds__(TPB) void k_nt_lin(NtRows a, int diag, double omega, double delta, double theta,
-                                                 double *Rw)
+// The control block of a diagonal Newton solve, whose loop is tested on the device:
+// the host enqueues iterations ahead and reads this once per batch of them.  With a
+// read-back of the merit's partial sums an iteration each took 70 us at 64000 rows,
+// 43 us of them on the device; @@FIG@@
+struct NtCtl {
+  static const int RING = 64;
+  int done, iters, nan;
+  double merit;
+  double hist[RING];     // merit of iteration k at k % RING
+};
+
+struct NtTest {
+  NtCtl *ctl;            // null: no test
+  int k;                 // iterations before this launch
+  const double *part;    // the merit's partial sums after them
+  int np, maxiter;
+  double lo, meritval;
+};
+
+// the test of the loop after iteration k (nts.c:1199-1223), taken by every
+// workgroup alike from the same sums; workgroup 0 keeps the record.  True when the
+// loop has ended.
+__device__ __forceinline__ bool nt_test(const NtTest &t)
 {
+  __shared__ int ended;
+  double s = 0.0, z1 = 0.0, z2 = 0.0;
+  for (int k = threadIdx.x; k < t.np; k += TPB) s += t.part[k];
+  block_sum3(s, z1, z2);
+  if (threadIdx.x == 0)
+  {
+    // the loop's end in an earlier launch; one that workgroup 0 of this launch has
+    // written already is what this workgroup finds as well
+    int done = __hip_atomic_load(&t.ctl->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (!done && t.k > 0)
+    {
+      const double merit = 0.5*s/t.lo;
+      const int nan = merit != merit;
+      done = nan || t.k >= t.maxiter || !(merit > t.meritval);
+      if (blockIdx.x == 0)
+      {
+        t.ctl->merit = merit;
+        t.ctl->nan = nan;
+        if (!nan) { t.ctl->iters = t.k; t.ctl->hist[(t.k - 1) % NtCtl::RING] = merit; }
+        if (done) __hip_atomic_store(&t.ctl->done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    ended = done;
+  }
+  __syncthreads();
+  return ended != 0;
+}
+
+__global__ __launch_bounds__(TPB) void k_nt_lin(NtRows a, int diag, double omega, double delta, double theta,
+                                                 double *Rw, NtTest test)
+{
+  if (test.ctl && nt_test(test)) return;
   const int p = blockIdx.x*blockDim.x + threadIdx.x;
   if (p >= a.n) return;
   const int n = a.n;
@@ -447,6 +500,7 @@ struct NtWork {
 void sfgs_newton_release(sfgs_ctx *ctx)
 {
   release(ctx->nt_mem);
+  release(ctx->nt_ctl);
 }
 
 extern "C" {
@@ -536,25 +590,55 @@ int SFGS_Newton_Solve(sfgs_ctx *ctx, const SFGS_NEWTON_PARAM *par, double *merhi
   CHK(merit_of(merit));
   int iters = 0, nan = 0;
   const bool diag = par->linver == SFGS_NT_DIAG;
-  while (iters < par->maxiter && (diag || wk.matvecs < par->maxmatvec) && merit > par->meritval)
+  if (diag && iters < par->maxiter && merit > par->meritval && n > 0)
+  {
+    // batches of iterations without a read-back: 4, 8, 16, 32, 32, ...; what is
+    // enqueued past the loop's end returns at once
+    CHK(ensure(ctx, ctx->nt_ctl, sizeof(NtCtl)));
+    NtCtl *ctl = (NtCtl*)ctx->nt_ctl.p, h;
+    std::memset(&h, 0, sizeof(h));
+    HIPCHK(hipMemcpyAsync(ctl, &h, sizeof(h), hipMemcpyHostToDevice, st));
+    const double lo = ctx->energy < DBL_EPSILON ? 1.0 : ctx->energy;
+    NtTest test{ctl, 0, ctx->mpartials.p, 0, par->maxiter, lo, par->meritval};
+    for (int batch = 4; !h.done; batch = std::min(2*batch, NtCtl::RING/2))
+    {
+      const int last = (int)std::min((long long)test.k + batch, (long long)par->maxiter + 1);
+      for (; test.k < last; test.k ++)
+      {
+        hipLaunchKernelGGL(k_nt_lin, dim3(nblk(n)), dim3(TPB), 0, st, rows, 1, par->omega, delta, par->theta, ctx->R.p,
+                           test);
+        HIPCHK(hipGetLastError());
+        if (test.k == par->maxiter) continue;   // the last launch only tests
+        if (par->bodyspace) CHK(bodyspace_product(ctx, ctx->R.p, 4, 1, nullptr, nullptr, 0.0, 0.0, 0.0, nullptr));
+        CHK(launch_merit(ctx, par->bodyspace ? 0 : 1, nullptr, &ctl->done, &test.np));
+      }
+      HIPCHK(hipMemcpyAsync(&h, ctl, sizeof(h), hipMemcpyDeviceToHost, st));
+      HIPCHK(hipStreamSynchronize(st));
+      for (; iters < h.iters; iters ++)
+      {
+        if (merhist) merhist[iters] = h.hist[iters % NtCtl::RING];
+        if (mvhist) mvhist[iters] = 0;
+      }
+    }
+    merit = h.merit;
+    nan = h.nan;
+  }
+  while (!diag && iters < par->maxiter && wk.matvecs < par->maxmatvec && merit > par->meritval)
   {
     if (n > 0)
-      hipLaunchKernelGGL(k_nt_lin, dim3(nblk(n)), dim3(TPB), 0, st, rows, diag ? 1 : 0, par->omega, delta, par->theta,
-                         ctx->R.p);
+      hipLaunchKernelGGL(k_nt_lin, dim3(nblk(n)), dim3(TPB), 0, st, rows, 0, par->omega, delta, par->theta, ctx->R.p,
+                         NtTest{});
     HIPCHK(hipGetLastError());
-    if (!diag)
-    {
-      double bb = 0.0;
-      CHK(wk.dot(wk.b, wk.b, bb));
-      CHK(wk.gmres(wk.b, wk.dr, par->linmaxiter, 1, par->epsilon*std::sqrt(bb)));
-      if (n > 0)
-        hipLaunchKernelGGL(k_nt_update, dim3(nblk(n)), dim3(TPB), 0, st, n, ctx->R.p, wk.dr, ctx->pfri.p, ctx->pcoh.p);
-      HIPCHK(hipGetLastError());
-    }
+    double bb = 0.0;
+    CHK(wk.dot(wk.b, wk.b, bb));
+    CHK(wk.gmres(wk.b, wk.dr, par->linmaxiter, 1, par->epsilon*std::sqrt(bb)));
+    if (n > 0)
+      hipLaunchKernelGGL(k_nt_update, dim3(nblk(n)), dim3(TPB), 0, st, n, ctx->R.p, wk.dr, ctx->pfri.p, ctx->pcoh.p);
+    HIPCHK(hipGetLastError());
     CHK(merit_of(merit));
     if (std::isnan(merit)) { nan = 1; break; }
     if (merhist) merhist[iters] = merit;
-    if (mvhist) mvhist[iters] = diag ? 0 : wk.matvecs;
+    if (mvhist) mvhist[iters] = wk.matvecs;
     iters ++;
   }
   int singular = 0;

@@ -421,8 +421,8 @@ __device__ __forceinline__ bool sweep_slice(const SweepArgs<T> &a, int s, bool v
 // standalone merit (MERIT_Function with update_U, mrf.c:35-184) on the
 // canonical R buffer; one launch over all slices
 struct MeritArgs {
-  const int *row0, *nrows, *rowlen, *rowoff, *slen;
-  const long long *off;
+  const SliceTab *tab;
+  const int *rowlen, *rowoff;
   const double *W;
   const int *wcol;
   const double *Wd, *A, *B, *fri, *coh, *shift;
@@ -431,62 +431,64 @@ struct MeritArgs {
   int n, update_U;
   double *mpartials;
   double *conmerit;   // may be null: per-row C'AC (colour-major)
+  const int *stop;    // may be null: nonzero leaves everything as it is
 };
 
 // merit terms C'AC of the rows of one slice, added to up (lane g = 0 of each
-// row); lds: this wavefront's Gather<double>::LDS1 values
+// row); lds: this wavefront's Gather<double>::LDS1 values.  A wavefront's time is
+// its chain of loads, so the slice comes as one table entry and the row's data but
+// for A go out ahead of the gather: @@FIG@@
 template <int G>
 __device__ __forceinline__ void merit_slice(const MeritArgs &a, int s, bool valid, double &up, double *lds)
 {
   const int l = threadIdx.x & 63, r = l / G, g = l % G;
   const int n = a.n;
-  int nr = 0, r0 = 0, total = 0;
-  long long off = 0;
+  if (!__builtin_amdgcn_readfirstlane(valid)) return;
   s = __builtin_amdgcn_readfirstlane(s);
-  if (__builtin_amdgcn_readfirstlane(valid))
-  {
-    nr = a.nrows[s]; r0 = a.row0[s];
-    if (a.update_U) { off = a.off[s]; total = a.slen[s]; }
-  }
+  const SliceTab tab = a.tab[s];
+  const int stopped = a.stop ? *a.stop : 0;
+  const int nr = __builtin_amdgcn_readfirstlane(tab.nrows), r0 = __builtin_amdgcn_readfirstlane(tab.row0);
+  const int total = __builtin_amdgcn_readfirstlane(tab.blocks);
+  const long long off = (long long)__builtin_amdgcn_readfirstlane((int)(tab.off >> 32)) << 32 |
+                        (unsigned)__builtin_amdgcn_readfirstlane((int)tab.off);
+  if (__builtin_amdgcn_readfirstlane(stopped)) return;
   const bool act = r < nr;
-  const int p = act ? r0 + r : 0;
-  int len = 0, rs = 0;
-  if (total > 0) { len = a.rowlen[p]; rs = a.rowoff[p]; }
-  // the sweep's multiply-adds (sweep_slice), so that U equals the fused merit pass's
-  double u[3], none[3];
-  gather_rows<double, G, false, false, 4>(a.W, a.wcol, off, total, rs, len, act, a.R, a.R, 0, 0, lds, u, none);
-  if (act)
+  const int p = r0 + min(r, nr - 1), rs = a.rowoff[p], len = a.rowlen[p];
+  double R[3], Wi[9], Bv[3], U[3], fri = a.fri[p], coh = a.coh[p], shift = a.shift[p];
+  load3<false, 4>(a.R, p, R);
+  if (a.update_U)
   {
-    double R[3] = {a.R[4*(size_t)p], a.R[4*(size_t)p + 1], a.R[4*(size_t)p + 2]}, U[3];
-    if (a.update_U)
-    {
-      double Wi[9], Bv[3] = {a.B[p], a.B[(size_t)n + p], a.B[2*(size_t)n + p]};
 #pragma unroll
-      for (int e = 0; e < 9; e ++) Wi[e] = a.Wd[(size_t)e*n + p];
-      mv_add(Bv, Wi, R, U);
-      U[0] += u[0]; U[1] += u[1]; U[2] += u[2];
-      if (g == 0)
+    for (int k = 0; k < 3; k ++) Bv[k] = a.B[(size_t)k*n + p];
 #pragma unroll
-        for (int k = 0; k < 3; k ++) a.U[(size_t)k*n + p] = U[k];
-    }
-    else
-    {
+    for (int e = 0; e < 9; e ++) Wi[e] = a.Wd[(size_t)e*n + p];
+    // the sweep's multiply-adds (sweep_slice), so that U equals the fused merit pass's
+    double u[3], none[3];
+    gather_rows<double, G, false, false, 4>(a.W, a.wcol, off, total, rs, len, act, a.R, a.R, 0, 0, lds, u, none);
+    mv_add(Bv, Wi, R, U);
+    U[0] += u[0]; U[1] += u[1]; U[2] += u[2];
+    if (act && g == 0)
 #pragma unroll
-      for (int k = 0; k < 3; k ++) U[k] = a.U[(size_t)k*n + p];
-    }
-    double C[3], Ai[9];
-    merit_residual(a.fri[p], a.coh[p], a.shift[p], U, R, C);
+      for (int k = 0; k < 3; k ++) a.U[(size_t)k*n + p] = U[k];
+  }
+  else
+  {
 #pragma unroll
-    for (int e = 0; e < 9; e ++) Ai[e] = a.A[(size_t)e*n + p];
-    const double q0 = Ai[0]*C[0] + Ai[3]*C[1] + Ai[6]*C[2];
-    const double q1 = Ai[1]*C[0] + Ai[4]*C[1] + Ai[7]*C[2];
-    const double q2 = Ai[2]*C[0] + Ai[5]*C[1] + Ai[8]*C[2];
-    if (g == 0)
-    {
-      const double t = q0*C[0] + q1*C[1] + q2*C[2];
-      up += t;
-      if (a.conmerit) a.conmerit[p] = t;
-    }
+    for (int k = 0; k < 3; k ++) U[k] = a.U[(size_t)k*n + p];
+  }
+  if (!act) return;
+  double C[3], Ai[9];
+#pragma unroll
+  for (int e = 0; e < 9; e ++) Ai[e] = a.A[(size_t)e*n + p];
+  merit_residual(fri, coh, shift, U, R, C);
+  const double q0 = Ai[0]*C[0] + Ai[3]*C[1] + Ai[6]*C[2];
+  const double q1 = Ai[1]*C[0] + Ai[4]*C[1] + Ai[7]*C[2];
+  const double q2 = Ai[2]*C[0] + Ai[5]*C[1] + Ai[8]*C[2];
+  if (g == 0)
+  {
+    const double t = q0*C[0] + q1*C[1] + q2*C[2];
+    up += t;
+    if (a.conmerit) a.conmerit[p] = t;
   }
 }
 
