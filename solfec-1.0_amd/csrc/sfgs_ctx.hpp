@@ -117,6 +117,7 @@ struct sfgs_ctx {
   sfgs::DBuf<double> pen;                // penalty solve: spring, dashpot, hpow per contact, or the default six
   sfgs::DBuf<double> nt_mem;             // Newton solve: linearisation, Krylov vectors, partials
   sfgs::DBuf<unsigned char> nt_ctl;      // its control block (diagonal systems)
+  double *nt_host = nullptr;             // pinned: partials of a dot product and the residual estimate, written by kernels
   sfgs::DBuf<unsigned char> bar_mem;     // barrier schedule: colour tables, partials, counter
 
   // ---- reductions / control

@@ -18,10 +18,11 @@
 //                host in block order)
 //   k_nt_axpy, k_nt_scale, k_nt_precond, k_nt_update  the vector work of
 //                flexible GMRES (ext/krylov/flexgmres.c) and R = proj(R + dr)
-// The GMRES driver runs on the host: its Hessenberg matrix is at most 21 x 20
-// and every dot product is read back, as the reference's InnerProd returns a
-// value.  All of this is HBM-bound vector work (a W product streams the same
-// bytes as a sweep); the sweeps remain the solver of the hot path.
+// The diagonal solve runs its loop on the device (NtCtl); the GMRES driver runs on the
+// host, with the Arnoldi steps and the Hessenberg system (at most 21 x 20) on the
+// device and one wait per step for the residual estimate.  All of this is HBM-bound
+// vector work (a W product streams the same bytes as a sweep); the sweeps remain the
+// solver of the hot path.
 #include <hip/hip_runtime.h>
 #include <cmath>
 #include <cstring>
@@ -60,7 +61,8 @@ struct NtRows {
 // The control block of a diagonal Newton solve, whose loop is tested on the device:
 // the host enqueues iterations ahead and reads this once per batch of them.  With a
 // read-back of the merit's partial sums an iteration each took 70 us at 64000 rows,
-// 43 us of them on the device; @@FIG@@
+// 43 us of them on the device; now
+// 200 iterations take 9.6 ms on the device, the whole solve 12.0 ms in place of 15.4.
 struct NtCtl {
   static const int RING = 64;
   int done, iters, nan;
@@ -223,12 +225,6 @@ __global__ void k_nt_axpy(long long N, double alpha, const double *x, double *y)
   if (i < N) y[i] += alpha*x[i];
 }
 
-__global__ void k_nt_scale(long long N, double t, double *x)
-{
-  const long long i = (long long)blockIdx.x*blockDim.x + threadIdx.x;
-  if (i < N) x[i] *= t;
-}
-
 __global__ void k_nt_precond(int n, const double *P, const double *b, double *x)
 {
   const int p = blockIdx.x*blockDim.x + threadIdx.x;
@@ -261,35 +257,55 @@ struct NtScal {
   double rnorm;
 };
 
-// the sum of a dot product's block partials, in a fixed order; sqrt of it when root
-__global__ __launch_bounds__(TPB) void k_nt_dotfin(const double *part, int np, double *out, int root)
+// the sum of a dot product's block partials, in a fixed order, in all threads
+__device__ __forceinline__ double nt_dot_sum(const double *part, int np)
 {
+  __shared__ double sum;
   double v = threadIdx.x < np ? part[threadIdx.x] : 0.0, z1 = 0.0, z2 = 0.0;
   block_sum3(v, z1, z2);
-  if (threadIdx.x == 0) *out = root ? sqrt(v) : v;
+  if (threadIdx.x == 0) sum = v;
+  __syncthreads();
+  v = sum;
+  __syncthreads();   // before the slots' next use
+  return v;
 }
 
-// y += sign * (*alpha) x
-__global__ void k_nt_axpy_dev(long long N, const double *alpha, double sign, const double *x, double *y)
+// One modified Gram-Schmidt step: y -= h x0 with h the dot product whose partial
+// sums the launch before left in p0 (kept in *out; x0 null: no update), then the
+// partial sums of x1 . y (x1 null: of y . y) into p1.  A step is bound by its
+// launches (3 us each for 60k values), so the update, the sum of the partials and the
+// next product are one launch instead of three, the step's end one
+// instead of five, and what the host needs is written to its memory: 11 linearisations of
+// 20011 contacts in body space with 62 steps took 10.6 ms and take 6.8.
+__global__ __launch_bounds__(TPB) void k_nt_mgs(long long N, const double *x0, const double *p0, double *out,
+                                                 const double *x1, double *y, double *p1)
 {
-  const long long i = (long long)blockIdx.x*blockDim.x + threadIdx.x;
-  if (i < N) y[i] += (sign*(*alpha))*x[i];
+  const double h = x0 ? nt_dot_sum(p0, gridDim.x) : 0.0, mh = -1.0*h;
+  if (x0 && blockIdx.x == 0 && threadIdx.x == 0) *out = h;
+  double s = 0.0, z1 = 0.0, z2 = 0.0;
+  for (long long i = (long long)blockIdx.x*TPB + threadIdx.x; i < N; i += (long long)gridDim.x*TPB)
+  {
+    double v = y[i];
+    if (x0) { v += mh*x0[i]; y[i] = v; }
+    s += (x1 ? x1[i] : v)*v;
+  }
+  block_sum3(s, z1, z2);
+  if (threadIdx.x == 0) p1[blockIdx.x] = s;
 }
 
-// x *= 1 / (*t) unless *t is 0
-__global__ void k_nt_scale_inv(long long N, const double *t, double *x)
+// x *= t, and *rs = r: the start of a cycle
+__global__ void k_nt_start(long long N, double t, double *x, double *rs, double r)
 {
   const long long i = (long long)blockIdx.x*blockDim.x + threadIdx.x;
-  const double tv = *t;
-  if (i < N && tv != 0.0) x[i] *= 1.0/tv;
+  if (i == 0) *rs = r;
+  if (i < N) x[i] *= t;
 }
 
 // column i - 1 of the Arnoldi step: the previous rotations, a new one, the
 // updated right-hand side and the residual estimate |rs[i]| (flexgmres.c:531-557)
-__global__ void k_nt_givens(NtScal *sc, int i)
+__device__ void nt_givens(NtScal *sc, int i)
 {
 #pragma clang fp contract(off)
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
   double *hh = sc->hh, *c = sc->c, *s = sc->s, *rs = sc->rs, t;
 #define HH(a, b) hh[(a)*NT_KDIM + (b)]
   for (int j = 1; j < i; j ++)
@@ -312,18 +328,65 @@ __global__ void k_nt_givens(NtScal *sc, int i)
 #undef HH
 }
 
+// the end of Arnoldi step i: its norm from the partial sums of the launch before, y
+// scaled by it (unless it is 0), and in workgroup 0 the Givens update; the residual
+// estimate goes to the host's memory
+__global__ __launch_bounds__(TPB) void k_nt_arnoldi(long long N, const double *part, int np, double *y, NtScal *sc, int i,
+                                                     double *rnorm)
+{
+  const double t = sqrt(nt_dot_sum(part, np));
+  if (t != 0.0)
+    for (long long k = (long long)blockIdx.x*TPB + threadIdx.x; k < N; k += (long long)gridDim.x*TPB) y[k] *= 1.0/t;
+  if (blockIdx.x == 0 && threadIdx.x == 0)
+  {
+    sc->hh[i*NT_KDIM + i - 1] = t;
+    nt_givens(sc, i);
+    *rnorm = sc->rnorm;
+  }
+}
+
+// the end of a cycle of m steps: back-substitution in the Hessenberg system (every
+// workgroup for itself; hh and rs stay as they are) and x += sum_j rs_j pre_j
+__global__ __launch_bounds__(TPB) void k_nt_cycle(long long N, const NtScal *sc, int m, const double *pre, double *x)
+{
+  __shared__ double hh[(NT_KDIM + 1)*NT_KDIM], rs[NT_KDIM + 1];
+  for (int k = threadIdx.x; k < m*NT_KDIM; k += TPB) hh[k] = sc->hh[k];
+  if (threadIdx.x < m) rs[threadIdx.x] = sc->rs[threadIdx.x];
+  __syncthreads();
+  if (threadIdx.x == 0)
+  {
+#pragma clang fp contract(off)
+    rs[m - 1] = rs[m - 1]/hh[(m - 1)*NT_KDIM + m - 1];
+    for (int k = m - 2; k >= 0; k --)
+    {
+      double t = 0.0;
+      for (int j = k + 1; j < m; j ++) t -= hh[k*NT_KDIM + j]*rs[j];
+      t += rs[k];
+      rs[k] = t/hh[k*NT_KDIM + k];
+    }
+  }
+  __syncthreads();
+  for (long long i = (long long)blockIdx.x*TPB + threadIdx.x; i < N; i += (long long)gridDim.x*TPB)
+  {
+    // explicit multiply-adds: the sums of one vector update after the other
+#pragma clang fp contract(off)
+    double w = pre[(size_t)(m - 1)*N + i]*rs[m - 1];
+    for (int j = m - 2; j >= 0; j --) w = fma(rs[j], pre[(size_t)j*N + i], w);
+    x[i] += w;
+  }
+}
+
 // the device vectors of one Newton solve
 struct NtWork {
   sfgs_ctx *ctx;
   int n;
   long long N;
-  double *X, *Y, *P, *b, *dr, *R0, *kry, *pre, *w, *r, *part;
+  double *X, *Y, *P, *b, *dr, *R0, *kry, *pre, *r, *part;
   NtScal *sc;
   NtMat mat;
   int bodyspace = 0;
   int matvecs = 0;
-  std::vector<double> hpart;
-  double rs0 = 0.0, rnorm_h = 0.0;   // host ends of the small copies
+  double *hpart;             // in host memory that kernels write: partials of a dot product, a residual estimate
 
   double *kv(int k) const { return kry + (size_t)k*N; }
   double *pv(int k) const { return pre + (size_t)k*N; }
@@ -345,11 +408,13 @@ struct NtWork {
     return 0;
   }
 
+  int dot_grid() const { return std::max(1, std::min(NT_DOT_BLOCKS, nblk(N))); }
+
+  // the partial sums straight into host memory: one wait, no copy
   int dot(const double *a, const double *b2, double &out)
   {
-    const int grid = std::max(1, std::min(NT_DOT_BLOCKS, nblk(N)));
-    hipLaunchKernelGGL(k_nt_dot, dim3(grid), dim3(TPB), 0, ctx->stream, N, a, b2, part);
-    HIPCHK(hipMemcpyAsync(hpart.data(), part, sizeof(double)*(size_t)grid, hipMemcpyDeviceToHost, ctx->stream));
+    const int grid = dot_grid();
+    hipLaunchKernelGGL(k_nt_dot, dim3(grid), dim3(TPB), 0, ctx->stream, N, a, b2, hpart);
     HIPCHK(hipStreamSynchronize(ctx->stream));
     double s = 0.0;
     for (int k = 0; k < grid; k ++) s += hpart[k];
@@ -357,32 +422,23 @@ struct NtWork {
     return 0;
   }
 
-  // x'y (or its square root) into device memory: no read-back
-  void dot_dev(const double *a, const double *b2, double *out, int root)
+  // modified Gram-Schmidt of kv(i) against kv(0) .. kv(i - 1), column i - 1 of the
+  // Hessenberg matrix, and the Givens update
+  void arnoldi(int i)
   {
-    const int grid = std::max(1, std::min(NT_DOT_BLOCKS, nblk(N)));
-    hipLaunchKernelGGL(k_nt_dot, dim3(grid), dim3(TPB), 0, ctx->stream, N, a, b2, part);
-    hipLaunchKernelGGL(k_nt_dotfin, dim3(1), dim3(TPB), 0, ctx->stream, part, grid, out, root);
-  }
-
-  void axpy_dev(const double *alpha, double sign, const double *x, double *y)
-  {
-    if (N > 0) hipLaunchKernelGGL(k_nt_axpy_dev, dim3(nblk(N)), dim3(TPB), 0, ctx->stream, N, alpha, sign, x, y);
-  }
-
-  void scale_inv_dev(const double *t, double *x)
-  {
-    if (N > 0) hipLaunchKernelGGL(k_nt_scale_inv, dim3(nblk(N)), dim3(TPB), 0, ctx->stream, N, t, x);
+    const int grid = dot_grid();
+    double *p[2] = {part, part + NT_DOT_BLOCKS}, *y = kv(i);
+    for (int j = 0; j <= i; j ++)
+      hipLaunchKernelGGL(k_nt_mgs, dim3(grid), dim3(TPB), 0, ctx->stream, N, j > 0 ? kv(j - 1) : (const double *)nullptr,
+                         (const double *)p[(j + 1) & 1], sc->hh + (j > 0 ? j - 1 : 0)*NT_KDIM + i - 1,
+                         j < i ? kv(j) : (const double *)nullptr, y, p[j & 1]);
+    hipLaunchKernelGGL(k_nt_arnoldi, dim3(grid), dim3(TPB), 0, ctx->stream, N, (const double *)p[i & 1], grid, y, sc, i,
+                       hpart + NT_DOT_BLOCKS);
   }
 
   void axpy(double alpha, const double *x, double *y)
   {
     if (N > 0) hipLaunchKernelGGL(k_nt_axpy, dim3(nblk(N)), dim3(TPB), 0, ctx->stream, N, alpha, x, y);
-  }
-
-  void scale(double t, double *x)
-  {
-    if (N > 0) hipLaunchKernelGGL(k_nt_scale, dim3(nblk(N)), dim3(TPB), 0, ctx->stream, N, t, x);
   }
 
   int copy(const double *x, double *y)
@@ -401,18 +457,17 @@ struct NtWork {
   // device (dot products reduced there, the Givens update in one thread); the
   // host reads the residual estimate once per iteration and the small
   // Hessenberg system once per cycle.
-  int gmres(const double *bb, double *x, int max_iter, int min_iter, double a_tol)
+  // bnorm2: bb . bb
+  int gmres(const double *bb, double bnorm2, double *x, int max_iter, int min_iter, double a_tol)
   {
     const int k_dim = NT_KDIM;
     NtScal h;
     double r_norm, b_norm, t;
     int iter = 0, i = 0;
-    double *hh = sc->hh;
-#define HHD(a, b) (hh + (a)*NT_KDIM + (b))
 #define HHH(a, b) h.hh[(a)*NT_KDIM + (b)]
     CHK(copy(bb, kv(0)));
     CHK(matvec(-1.0, x, 1.0, kv(0)));
-    CHK(dot(bb, bb, t)); b_norm = std::sqrt(t);
+    b_norm = std::sqrt(bnorm2);
     if (b_norm != 0.0 && !std::isfinite(b_norm)) return 0;   // non-finite input: x untouched
     CHK(dot(kv(0), kv(0), t)); r_norm = std::sqrt(t);
     if (r_norm != 0.0 && !std::isfinite(r_norm)) return 0;
@@ -427,45 +482,24 @@ struct NtWork {
         CHK(dot(r, r, t)); r_norm = std::sqrt(t);
         if (r_norm <= epsilon) break;
       }
-      rs0 = r_norm;   // rs[0] of the cycle
-      HIPCHK(hipMemcpyAsync(sc->rs, &rs0, sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-      scale(1.0/r_norm, kv(0));
+      hipLaunchKernelGGL(k_nt_start, dim3(nblk(std::max(N, 1LL))), dim3(TPB), 0, ctx->stream, N, 1.0/r_norm, kv(0), sc->rs,
+                         r_norm);
       i = 0;
       while (i < k_dim && iter < max_iter)
       {
         i ++;
         iter ++;
-        HIPCHK(hipMemsetAsync(pv(i - 1), 0, sizeof(double)*(size_t)N, ctx->stream));
         precond(kv(i - 1), pv(i - 1));
         CHK(matvec(1.0, pv(i - 1), 0.0, kv(i)));
-        for (int j = 0; j < i; j ++)   // modified Gram-Schmidt
-        {
-          dot_dev(kv(j), kv(i), HHD(j, i - 1), 0);
-          axpy_dev(HHD(j, i - 1), -1.0, kv(j), kv(i));
-        }
-        dot_dev(kv(i), kv(i), HHD(i, i - 1), 1);
-        scale_inv_dev(HHD(i, i - 1), kv(i));
-        hipLaunchKernelGGL(k_nt_givens, dim3(1), dim3(64), 0, ctx->stream, sc, i);
-        HIPCHK(hipMemcpyAsync(&rnorm_h, &sc->rnorm, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+        arnoldi(i);
         HIPCHK(hipStreamSynchronize(ctx->stream));
-        r_norm = rnorm_h;
+        r_norm = hpart[NT_DOT_BLOCKS];
         if (r_norm <= epsilon && iter >= min_iter) break;
       }
-      HIPCHK(hipMemcpyAsync(&h, sc, sizeof(NtScal), hipMemcpyDeviceToHost, ctx->stream));
-      HIPCHK(hipStreamSynchronize(ctx->stream));
+      const int m = i;
+      hipLaunchKernelGGL(k_nt_cycle, dim3(dot_grid()), dim3(TPB), 0, ctx->stream, N, (const NtScal *)sc, m,
+                         (const double *)pre, x);
       HIPCHK(hipGetLastError());
-      h.rs[i - 1] = h.rs[i - 1]/HHH(i - 1, i - 1);
-      for (int k = i - 2; k >= 0; k --)
-      {
-        t = 0.0;
-        for (int j = k + 1; j < i; j ++) t -= HHH(k, j)*h.rs[j];
-        t += h.rs[k];
-        h.rs[k] = t/HHH(k, k);
-      }
-      CHK(copy(pv(i - 1), w));
-      scale(h.rs[i - 1], w);
-      for (int j = i - 2; j >= 0; j --) axpy(h.rs[j], pv(j), w);
-      axpy(1.0, w, x);
       if (r_norm <= epsilon && iter >= min_iter)
       {
         CHK(copy(bb, r));
@@ -474,6 +508,18 @@ struct NtWork {
         if (r_norm <= epsilon) break;
         CHK(copy(r, kv(0)));   // false convergence
         i = 0;
+      }
+      if (iter >= max_iter) break;
+      // a restart: the residual from the Krylov vectors
+      HIPCHK(hipMemcpyAsync(&h, sc, sizeof(NtScal), hipMemcpyDeviceToHost, ctx->stream));
+      HIPCHK(hipStreamSynchronize(ctx->stream));
+      h.rs[m - 1] = h.rs[m - 1]/HHH(m - 1, m - 1);
+      for (int k = m - 2; k >= 0; k --)
+      {
+        t = 0.0;
+        for (int j = k + 1; j < m; j ++) t -= HHH(k, j)*h.rs[j];
+        t += h.rs[k];
+        h.rs[k] = t/HHH(k, k);
       }
       for (int j = i; j > 0; j --)
       {
@@ -488,7 +534,6 @@ struct NtWork {
         axpy(1.0, kv(i), kv(0));
       }
     }
-#undef HHD
 #undef HHH
     HIPCHK(hipGetLastError());
     return 0;
@@ -501,6 +546,8 @@ void sfgs_newton_release(sfgs_ctx *ctx)
 {
   release(ctx->nt_mem);
   release(ctx->nt_ctl);
+  if (ctx->nt_host) (void)hipHostFree(ctx->nt_host);
+  ctx->nt_host = nullptr;
 }
 
 extern "C" {
@@ -523,19 +570,20 @@ int SFGS_Newton_Solve(sfgs_ctx *ctx, const SFGS_NEWTON_PARAM *par, double *merhi
   const long long N = 3LL*n;
   const size_t N1 = (size_t)std::max(N, 1LL), n1 = (size_t)std::max(n, 1);
 
-  // one allocation: X, Y, P (9 per row), b, dr, w, r (3 per row), R0 (4 per
+  // one allocation: X, Y, P (9 per row), b, dr, r (3 per row), R0 (4 per
   // row), the Krylov and the preconditioned vectors, dot partials
   const size_t scal_words = (sizeof(NtScal) + 7)/8;
-  const size_t words = 27*n1 + 4*N1 + 4*n1 + (size_t)(2*NT_KDIM + 1)*N1 + NT_DOT_BLOCKS + scal_words;
+  const size_t words = 27*n1 + 3*N1 + 4*n1 + (size_t)(2*NT_KDIM + 1)*N1 + 2*NT_DOT_BLOCKS + scal_words;
   CHK(ensure(ctx, ctx->nt_mem, words));
   NtWork wk;
   double *m0 = ctx->nt_mem.p;
   wk.ctx = ctx; wk.n = n; wk.N = N;
-  wk.X = m0; wk.Y = wk.X + 9*n1; wk.P = wk.Y + 9*n1; wk.b = wk.P + 9*n1; wk.dr = wk.b + N1; wk.w = wk.dr + N1;
-  wk.r = wk.w + N1; wk.R0 = wk.r + N1; wk.kry = wk.R0 + 4*n1; wk.pre = wk.kry + (size_t)(NT_KDIM + 1)*N1;
+  wk.X = m0; wk.Y = wk.X + 9*n1; wk.P = wk.Y + 9*n1; wk.b = wk.P + 9*n1; wk.dr = wk.b + N1; wk.r = wk.dr + N1;
+  wk.R0 = wk.r + N1; wk.kry = wk.R0 + 4*n1; wk.pre = wk.kry + (size_t)(NT_KDIM + 1)*N1;
   wk.part = wk.pre + (size_t)NT_KDIM*N1;
-  wk.sc = (NtScal*)(wk.part + NT_DOT_BLOCKS);
-  wk.hpart.resize(NT_DOT_BLOCKS);
+  wk.sc = (NtScal*)(wk.part + 2*NT_DOT_BLOCKS);
+  if (!ctx->nt_host) HIPCHK(hipHostMalloc((void**)&ctx->nt_host, sizeof(double)*(NT_DOT_BLOCKS + 1), hipHostMallocDefault));
+  wk.hpart = ctx->nt_host;
   HIPCHK(hipMemsetAsync(m0, 0, sizeof(double)*words, st));
   if (n > 0) HIPCHK(hipMemcpyAsync(wk.R0, ctx->R.p, sizeof(double)*4*(size_t)n, hipMemcpyDeviceToDevice, st));
   CHK(ensure(ctx, ctx->failcount, 4));
@@ -631,7 +679,7 @@ int SFGS_Newton_Solve(sfgs_ctx *ctx, const SFGS_NEWTON_PARAM *par, double *merhi
     HIPCHK(hipGetLastError());
     double bb = 0.0;
     CHK(wk.dot(wk.b, wk.b, bb));
-    CHK(wk.gmres(wk.b, wk.dr, par->linmaxiter, 1, par->epsilon*std::sqrt(bb)));
+    CHK(wk.gmres(wk.b, bb, wk.dr, par->linmaxiter, 1, par->epsilon*std::sqrt(bb)));
     if (n > 0)
       hipLaunchKernelGGL(k_nt_update, dim3(nblk(n)), dim3(TPB), 0, st, n, ctx->R.p, wk.dr, ctx->pfri.p, ctx->pcoh.p);
     HIPCHK(hipGetLastError());
