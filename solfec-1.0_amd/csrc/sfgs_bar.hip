@@ -132,10 +132,10 @@ __global__ __launch_bounds__(BAR_NW*64) void k_bar(BarArgs<T> b)
       for (int s = s0 + L*BAR_NW + wave; s < s1; s += b.nwg*BAR_NW)
       {
         if (mer)
-          sweep_slice<T, G, true, true>(a, s, true, lo, hi, back, &sweepno, a.failkey, a.failcount, &b.ctrl->aborted,
+          sweep_slice<T, G, true, true>(a, a.tab, s, true, lo, hi, back, &sweepno, a.failkey, a.failcount, &b.ctrl->aborted,
                                         eu, el, up, lds);
         else
-          sweep_slice<T, G, false, true>(a, s, true, lo, hi, back, &sweepno, a.failkey, a.failcount,
+          sweep_slice<T, G, false, true>(a, a.tab, s, true, lo, hi, back, &sweepno, a.failkey, a.failcount,
                                          &b.ctrl->aborted, eu, el, up, lds);
       }
       if (ci == b.ncol - 1)

@@ -144,7 +144,7 @@ __device__ __forceinline__ bool batch_sweep(const BatchGeom &geo, const SweepArg
     if (s0 == s1) continue;   // same decision in every workgroup of the scene
     const int lo = back ? geo.gptr[gi + 1] : sc.row0, hi = back ? sc.row1 : geo.gptr[gi];
     for (int s = s0 + w*NW + wave; s < s1; s += nw*NW)
-      sweep_slice<T, G, MERIT>(a, s, true, lo, hi, back, sweepno, &o->failkey, &o->failcount, &o->aborted, eu, el, up,
+      sweep_slice<T, G, MERIT>(a, a.tab, s, true, lo, hi, back, sweepno, &o->failkey, &o->failcount, &o->aborted, eu, el, up,
                                lds);
     if (!scene_barrier(bar, nw, geo.abort_all, geo.spin_limit, flag)) return false;
   }
@@ -346,8 +346,8 @@ struct UScene {
 // list: per slice of the launch its number, its scene and the rows already updated
 // in this sweep (forward: the scene's earlier colours; backward: its later ones)
 template <typename T, int G, bool MERIT>
-__global__ __launch_bounds__(TPB) void k_usweep(SweepArgs<T> a, const int4 *list, int nlist, BatchOut *out,
-                                                double *spart, int backward)
+__global__ __launch_bounds__(TPB) void k_usweep(const int4 *list, BatchOut *out, const SliceTab *tabs, int nlist,
+                                                int backward, double *spart, SweepArgs<T> a)
 {
   const int idx = __builtin_amdgcn_readfirstlane(blockIdx.x*(TPB/SLICE) + (threadIdx.x >> 6));
   if (idx >= nlist) return;                       // whole wavefront
@@ -358,7 +358,7 @@ __global__ __launch_bounds__(TPB) void k_usweep(SweepArgs<T> a, const int4 *list
   double eu = 0.0, el = 0.0, up = 0.0;
   int sweepno = o->iters0 + o->sweeps;
   // a finished scene: whole wavefront
-  if (!sweep_slice<T, G, MERIT>(a, s, true, e.z, e.w, backward, &sweepno, &o->failkey, &o->failcount, &o->aborted,
+  if (!sweep_slice<T, G, MERIT>(a, tabs, s, true, e.z, e.w, backward, &sweepno, &o->failkey, &o->failcount, &o->aborted,
                                 eu, el, up, lds[threadIdx.x >> 6], &o->done)) return;
   eu = wave_sum(eu); el = wave_sum(el); up = wave_sum(up);
   if ((threadIdx.x & 63) == 0)
@@ -601,11 +601,11 @@ static int run_union(sfgs_ctx *ctx, const SFGS_PARAM *par, const BatchArgs<T> &b
           if (nl == 0) continue;
           const dim3 grid((nl + TPB/SLICE - 1) / (TPB/SLICE));
           if (merit)
-            hipLaunchKernelGGL((k_usweep<TT, G, true>), grid, dim3(TPB), 0, st, a,
-                               (back ? listb : listf) + cstart[c], nl, out, spart, back);
+            hipLaunchKernelGGL((k_usweep<TT, G, true>), grid, dim3(TPB), 0, st, (back ? listb : listf) + cstart[c],
+                               out, a.tab, nl, back, spart, a);
           else
-            hipLaunchKernelGGL((k_usweep<TT, G, false>), grid, dim3(TPB), 0, st, a,
-                               (back ? listb : listf) + cstart[c], nl, out, spart, back);
+            hipLaunchKernelGGL((k_usweep<TT, G, false>), grid, dim3(TPB), 0, st, (back ? listb : listf) + cstart[c],
+                               out, a.tab, nl, back, spart, a);
         }
         hipLaunchKernelGGL(k_uscene, dim3(nsc), dim3(TPB), 0, st, 1, usc, (const double*)spart, out, bound, miniter,
                            nomerit, eps, meritval, kk, ctx->u_active.p);

@@ -205,10 +205,10 @@ __global__ __launch_bounds__(64) void k_flow(FlowArgs<T> f)
       __atomic_signal_fence(__ATOMIC_SEQ_CST);
       // lower-colour neighbours (j < row0 <= p) are read from Q, the rest from P
       if (merit)
-        sweep_slice<T, G, true, true>(a, s, true, 0, row0, 0, f.sweepno, a.failkey, a.failcount, &f.ctrl->aborted,
+        sweep_slice<T, G, true, true>(a, a.tab, s, true, 0, row0, 0, f.sweepno, a.failkey, a.failcount, &f.ctrl->aborted,
                                       eu, el, up, lds);
       else
-        sweep_slice<T, G, false, true>(a, s, true, 0, row0, 0, f.sweepno, a.failkey, a.failcount, &f.ctrl->aborted,
+        sweep_slice<T, G, false, true>(a, a.tab, s, true, 0, row0, 0, f.sweepno, a.failkey, a.failcount, &f.ctrl->aborted,
                                        eu, el, up, lds);
       publish_fence();
       if (act && g == 0) cst(f.ver + row0 + r, k + 1);

@@ -730,21 +730,28 @@ __device__ __forceinline__ int xcd_block(int b, int nb)
 template <int NT = TPB>
 __device__ void finish_sweep(Ctrl *ctrl, const double *partials, int np, double *hist);
 
+// The slice table, the stop flag, the slices and nb come first: they are in registers
+// when a wavefront starts (the preloaded arguments of the Makefile), so that its table
+// entry is on the way while the other arguments are fetched; both are misses of 0.6 us in
+// a launch of 6 to 8.  us a sweep without and with: 1000 rows 71.9 and 70.6, 7919 rows
+// 88.0 and 85.3, 60001 ellipsoids 100.2 and 98.2, 200k 192.3 and 186.5, mixed 107.6 and
+// 105.7.
 // nb: the launch's workgroups (an argument: gridDim would be a load of its own).
 // fin (the last launch of a sweep only): the block that completes the launch
 // last takes the sweep's termination test, as k_finish would after it
 // WPB wavefronts per workgroup (one slice each)
 template <typename T, int G, bool MERIT, int WPB = TPB/SLICE>
-__global__ __launch_bounds__(WPB*64) void k_sweep(SweepArgs<T> a, int s0, int s1, int pbase, int upd_lo, int upd_hi,
-                                                   int backward, int xcd, int nb, int *fin, int np, double *hist)
+__global__ __launch_bounds__(WPB*64) void k_sweep(const SliceTab *tabs, const int *stop, int s0, int s1, int nb, int xcd,
+                                                   int pbase, int upd_lo, int upd_hi, int backward, int np, int *fin,
+                                                   double *hist, SweepArgs<T> a)
 {
   const int bx = xcd_block(blockIdx.x, nb), bb = xcd ? bx : (int)blockIdx.x;
   const int s = s0 + bb*WPB + (threadIdx.x >> 6);
   __shared__ T lds[WPB][MERIT ? Gather<T>::LDS2 : Gather<T>::LDS1];
   double eu = 0.0, el = 0.0, up = 0.0;
   // done is uniform: set only between launches, by the finish of an earlier sweep
-  if (!sweep_slice<T, G, MERIT>(a, s, s < s1, upd_lo, upd_hi, backward, &a.ctrl->sweeps, a.failkey, a.failcount,
-                                &a.ctrl->aborted, eu, el, up, lds[threadIdx.x >> 6], &a.ctrl->done)) return;
+  if (!sweep_slice<T, G, MERIT>(a, tabs, s, s < s1, upd_lo, upd_hi, backward, &a.ctrl->sweeps, a.failkey, a.failcount,
+                                &a.ctrl->aborted, eu, el, up, lds[threadIdx.x >> 6], stop)) return;
   block_sum3<WPB*64>(eu, el, up);
   if (threadIdx.x == 0)
   {
@@ -771,7 +778,7 @@ __global__ __launch_bounds__(WPB*64) void k_sweep(SweepArgs<T> a, int s0, int s1
 
 // Several consecutive colours of a sweep, each of at most a few slices, in one
 // launch of one workgroup: colour after colour in sweep order, wavefront w
-// taking slices w, w + NW, ... of each, with a workgroup barrier between
+// taking slice w of each, with a workgroup barrier between
 // colours.  The rows of a colour then read the reactions the colour before
 // wrote through the workgroup's own L1, which the barrier's workgroup-scope
 // fence makes visible: the same iterates as one launch per colour, one launch
@@ -784,18 +791,18 @@ struct ColourGroup {
 };
 
 template <typename T, int G, bool MERIT, int NW>
-__global__ __launch_bounds__(NW*64) void k_sweep_group(SweepArgs<T> a, ColourGroup cg, int pbase, int backward,
-                                                        int *fin, int np, double *hist)
+__global__ __launch_bounds__(NW*64) void k_sweep_group(const SliceTab *tabs, const int *stop, int pbase, int backward,
+                                                        int np, int *fin, double *hist, ColourGroup cg, SweepArgs<T> a)
 {
   const int w = threadIdx.x >> 6;
   __shared__ T lds[NW][MERIT ? Gather<T>::LDS2 : Gather<T>::LDS1];
   double eu = 0.0, el = 0.0, up = 0.0;
-  if (a.ctrl->done) return;
   for (int q = 0; q < cg.n; q ++)
   {
-    for (int s = cg.s0[q] + w; s < cg.s1[q]; s += NW)
-      sweep_slice<T, G, MERIT>(a, s, true, cg.lo[q], cg.hi[q], backward, &a.ctrl->sweeps, a.failkey, a.failcount,
-                               &a.ctrl->aborted, eu, el, up, lds[w]);
+    // at most NW slices; the stop flag, the same in all wavefronts, beside the table entry
+    const int s = cg.s0[q] + w;
+    if (!sweep_slice<T, G, MERIT>(a, tabs, s, s < cg.s1[q], cg.lo[q], cg.hi[q], backward, &a.ctrl->sweeps, a.failkey,
+                                  a.failcount, &a.ctrl->aborted, eu, el, up, lds[w], q == 0 ? stop : nullptr)) return;
     __syncthreads();   // this colour's reactions before the next colour's gathers
   }
   block_sum3<NW*64>(eu, el, up);
@@ -1913,12 +1920,15 @@ int SFGS_System_Upload(sfgs_ctx *ctx, int n, const int *rowptr, const int *col, 
 // one colour launch of k_sweep with the context's lanes per row and wavefronts per workgroup
 #define SFGS_SWEEP_WPB(MER, GG) \
   switch (ctx->wpb_run) { \
-  case 1: hipLaunchKernelGGL((k_sweep<T, GG, MER, 1>), dim3(grid[c]), dim3(64), 0, ctx->stream, a, ctx->h_cslice[c], \
-                             ctx->h_cslice[c + 1], pbase[c], lo, hi, backward, xcd, grid[c], f, np, hist); break; \
-  case 2: hipLaunchKernelGGL((k_sweep<T, GG, MER, 2>), dim3(grid[c]), dim3(128), 0, ctx->stream, a, ctx->h_cslice[c], \
-                             ctx->h_cslice[c + 1], pbase[c], lo, hi, backward, xcd, grid[c], f, np, hist); break; \
-  default: hipLaunchKernelGGL((k_sweep<T, GG, MER, 4>), dim3(grid[c]), dim3(256), 0, ctx->stream, a, ctx->h_cslice[c], \
-                              ctx->h_cslice[c + 1], pbase[c], lo, hi, backward, xcd, grid[c], f, np, hist); break; }
+  case 1: hipLaunchKernelGGL((k_sweep<T, GG, MER, 1>), dim3(grid[c]), dim3(64), 0, ctx->stream, a.tab, \
+                             &a.ctrl->done, ctx->h_cslice[c], ctx->h_cslice[c + 1], grid[c], xcd, pbase[c], lo, hi, backward, \
+                             np, f, hist, a); break; \
+  case 2: hipLaunchKernelGGL((k_sweep<T, GG, MER, 2>), dim3(grid[c]), dim3(128), 0, ctx->stream, a.tab, \
+                             &a.ctrl->done, ctx->h_cslice[c], ctx->h_cslice[c + 1], grid[c], xcd, pbase[c], lo, hi, backward, \
+                             np, f, hist, a); break; \
+  default: hipLaunchKernelGGL((k_sweep<T, GG, MER, 4>), dim3(grid[c]), dim3(256), 0, ctx->stream, a.tab, \
+                              &a.ctrl->done, ctx->h_cslice[c], ctx->h_cslice[c + 1], grid[c], xcd, pbase[c], lo, hi, backward, \
+                              np, f, hist, a); break; }
 #define SFGS_DISPATCH_SWEEP(MER) \
   switch (ctx->G_built) { \
   case 1: SFGS_SWEEP_WPB(MER, 1) break; \
@@ -1930,8 +1940,8 @@ int SFGS_System_Upload(sfgs_ctx *ctx, int n, const int *rowptr, const int *col, 
 // in its workgroup, and the most slices a colour may have to join it (one slice
 // per wavefront)
 #define SFGS_GROUP_LAUNCH(MER, GG) \
-  hipLaunchKernelGGL((k_sweep_group<T, GG, MER, GROUP_NW>), dim3(1), dim3(GROUP_NW*64), 0, ctx->stream, a, cg, \
-                     gslot, backward, f, np, hist);
+  hipLaunchKernelGGL((k_sweep_group<T, GG, MER, GROUP_NW>), dim3(1), dim3(GROUP_NW*64), 0, ctx->stream, \
+                     a.tab, &a.ctrl->done, gslot, backward, np, f, hist, cg, a);
 #define SFGS_DISPATCH_GROUP(MER) \
   switch (ctx->G_built) { \
   case 1: SFGS_GROUP_LAUNCH(MER, 1) break; \

@@ -263,10 +263,11 @@ __device__ __forceinline__ void gather_rows(const T *W, const int *wcol, long lo
 // the sweep number *sweepno, and raises *abortflag under FAILURE_EXIT.  The flag
 // is read together with the slice table, so both cost one memory round trip.
 // COH: P and Q are shared with other wavefronts of the same launch (r_ld / r_st).
+// tabs: a.tab, apart from a so that a kernel may have it among its first arguments.
 // lds: this wavefront's Gather<T>::LDS2 (merit) or LDS1 values.  s and valid are
 // the same in all lanes of the wavefront.
 template <typename T, int G, bool MERIT, bool COH = false>
-__device__ __forceinline__ bool sweep_slice(const SweepArgs<T> &a, int s, bool valid, int upd_lo, int upd_hi,
+__device__ __forceinline__ bool sweep_slice(const SweepArgs<T> &a, const SliceTab *tabs, int s, bool valid, int upd_lo, int upd_hi,
                                             int backward, const int *sweepno, unsigned long long *failkey,
                                             int *failcount, int *abortflag, double &eu, double &el, double &up,
                                             T *lds, const int *stop = nullptr)
@@ -275,7 +276,7 @@ __device__ __forceinline__ bool sweep_slice(const SweepArgs<T> &a, int s, bool v
   const int n = a.n;
   if (!__builtin_amdgcn_readfirstlane(valid)) return !(stop && *stop);
   s = __builtin_amdgcn_readfirstlane(s);
-  const SliceTab tab = a.tab[s];
+  const SliceTab tab = tabs[s];
   const int stopped = __builtin_amdgcn_readfirstlane(stop ? *stop : 0);
   const int nr = __builtin_amdgcn_readfirstlane(tab.nrows), r0 = __builtin_amdgcn_readfirstlane(tab.row0);
   const int total = __builtin_amdgcn_readfirstlane(tab.blocks);
