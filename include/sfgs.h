@@ -196,7 +196,7 @@ int SFGS_Set_Schedule(sfgs_ctx *ctx, int schedule);
 int SFGS_Set_Sweep_Block(sfgs_ctx *ctx, int waves_per_block);
 
 /* Order of the rows inside a colour (no counterpart in the reference): 0 =
- * decreasing row length (least slice padding); 1 = contact index; 2 = master
+ * decreasing row length; 1 = contact index; 2 = master
  * body in blocks of 64 bodies, then decreasing row length; 3 (default) = the
  * Z-order (Morton code on a 1024^3 grid over the bodies' bounding box) of the
  * master body's position, which keeps the rows of bodies close in space

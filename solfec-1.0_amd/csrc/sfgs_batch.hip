@@ -3,7 +3,7 @@
 //
 // The scenes share one device store: rows are ordered by (scene, colour,
 // -row length, i), so the rows of a scene form one contiguous range and each
-// (scene, colour) group one contiguous set of SELL-64 slices.  Scene s owns
+// (scene, colour) group one contiguous set of slices.  Scene s owns
 // workgroups [wg0, wg0 + nwg); they sweep the scene's colours in order, the
 // waves of the scene's workgroups taking the slices of a colour round robin,
 // and meet at a scene barrier after every colour.  A scene of one workgroup

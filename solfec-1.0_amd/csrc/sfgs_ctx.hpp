@@ -81,7 +81,7 @@ struct sfgs_ctx {
   std::vector<int> h_colptr, h_cslice;   // rows / slices per colour (host)
   sfgs::DBuf<unsigned char> scratch;     // hipcub temporary storage
 
-  // ---- slices (64/G rows of one colour each, colour-major)
+  // ---- slices (up to 64/G rows of one colour each, colour-major)
   int nslices = 0;
   sfgs::DBuf<int> slice_row0, slice_nrows, slice_len;   // slice_len: blocks of the slice
   sfgs::DBuf<long long> slice_off;       // block offset of slice (in blocks, multiple of 64)

@@ -6,7 +6,7 @@
 //  * colour-major order (row p = iperm[i]): rows sorted by (colour, -row length,
 //    i); per-row scalars in SoA planes (Wd[e*n + p], B[k*n + p], U[k*n + p]),
 //    reactions R as 4 doubles per row (32-byte aligned gathers);
-//  * off-diagonal blocks in slices: a slice is 64/G consecutive rows of one
+//  * off-diagonal blocks in slices: a slice is up to 64/G consecutive rows of one
 //    colour (one wavefront, G lanes per row), its blocks row after row without
 //    gaps; block q = 64 m + l of the slice stores element e at
 //    W[9*off + (9m + e)*64 + l] and the neighbour's row at wcol[off + q], so each
@@ -2152,7 +2152,7 @@ int SFGS_Solve(sfgs_ctx *ctx, const SFGS_PARAM *par, double *rerhist, double *me
   // the barrier schedule: one persistent launch, a device-wide barrier per colour
   const bool bar = ctx->schedule == 3 && n > 0 && ctx->G_built <= 2;
 
-  // wavefronts per workgroup: the FP64 sweeps (239 VGPRs, two wavefronts per
+  // wavefronts per workgroup: the FP64 sweeps (220 VGPRs, two wavefronts per
   // SIMD) run faster in workgroups of 2, the FP32 ones in workgroups of 4
   ctx->wpb_run = ctx->wpb ? ctx->wpb : (mixed ? 4 : 2);
   GsPlan pl;

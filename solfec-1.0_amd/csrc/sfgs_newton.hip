@@ -4,7 +4,7 @@
 // step), then the Gauss-Seidel solve as the fallback of an unconverged run.
 //
 // Vectors of the Newton step are 3 doubles per row in the colour-major row
-// order of the store, so the W products reuse the SELL-64 slices the sweeps
+// order of the store, so the W products reuse the slices the sweeps
 // stream.  The kernels:
 //   k_nt_lin     per row: C(U, R), X = dC/dU, Y = dC/dR of the smoothed cone
 //                residual (scf.c:28-133), b = -C, T = X W_ii + Y

@@ -256,7 +256,7 @@ __device__ __forceinline__ void gather_rows(const T *W, const int *wcol, long lo
   for (int c = 0; c < 3; c ++) { b[c] = gsum<G>(b[c]); if (TWO) u[c] = gsum<G>(u[c]); }
 }
 
-// One slice (64/G rows of one colour, one wavefront) of a sweep; false when *stop
+// One slice (up to 64/G rows of one colour, one wavefront) of a sweep; false when *stop
 // (a solve that has stopped; null: none) left it untouched.  eu, el and
 // up receive this lane's contributions to the error sums and to the merit
 // numerator.  A failed local solve is recorded in failkey / failcount, keyed by
