@@ -33,10 +33,10 @@ template <> __device__ __forceinline__ float fdiv<float>(float a, float b) { ret
 template <typename T> __device__ __forceinline__ T fsqrt(T x) { return sqrt(x); }
 template <> __device__ __forceinline__ float fsqrt<float>(float x) { return __builtin_amdgcn_sqrtf(x); }
 
-// 1/x and 1/sqrt(x) in FP64 for normal x (rsqrt64: positive), from the hardware
-// estimates by Newton's iteration, to about one ulp: the estimates are good to
-// 2^-22 or better, so two steps reach 2^-53.  The caller excludes zero,
-// subnormal and infinite arguments.
+// 1/x and 1/sqrt(x) in FP64 for normal x (rsqrt64: positive), to about one ulp:
+// the hardware estimates are good to 2^-22 or better, so two steps of Newton's
+// iteration (rcp64) or of Goldschmidt's coupled one (rsqrt64) reach 2^-53.  An
+// infinite or NaN argument gives NaN; the caller excludes zero and subnormal ones.
 __device__ __forceinline__ double rcp64(double x)
 {
   double r = __builtin_amdgcn_rcp(x);
@@ -224,21 +224,24 @@ __device__ __forceinline__ void scf_residual(T fri, T coh, T shift, const T *U, 
 // quotients shared (1/(1 + mu^2) once, |U_T| and 1/|S_T| from one reciprocal root
 // each) instead of three roots and five divisions, which took 920 of a slice's
 // clocks.  A tangential part whose square is subnormal counts as none: u2 = (1, 0)
-// as in spectral.  Only the merit sums depend on it.
+// as in spectral.  What is not finite stays so, as there: 0.5 (|l| + l) carries a NaN
+// and makes one of -inf where a maximum would give 0, and a tangential part that is
+// NaN or whose square overflows is NaN and not none.  Only the merit sums depend on it.
 __device__ __forceinline__ void merit_residual(double fri, double coh, double shift, const double *U, const double *R,
                                                double *C)
 {
   const double io = rcp64(1.0 + fri*fri);
   const double uu = U[0]*U[0] + U[1]*U[1];
-  const double ulen = uu >= DBL_MIN ? uu*rsqrt64(uu) : 0.0;
+  const double ulen = uu < DBL_MIN ? 0.0 : uu*rsqrt64(uu);
   const double F2 = U[2] + shift + fri*ulen;
   const double S0 = R[0] - U[0], S1 = R[1] - U[1], S2 = R[2] - F2 + coh;
   const double ss = S0*S0 + S1*S1;
-  const bool on = ss >= DBL_MIN;
-  const double is = on ? rsqrt64(ss) : 0.0, sl = ss*is;
-  const double g1 = fmax(-(S2 + fri*sl), 0.0)*io, g2 = fmax(sl - fri*S2, 0.0)*io;
+  const bool none = ss < DBL_MIN;
+  const double is = none ? 0.0 : rsqrt64(ss), sl = ss*is;
+  const double l1 = -(S2 + fri*sl)*io, l2 = (sl - fri*S2)*io;
+  const double g1 = 0.5*(fabs(l1) + l1), g2 = 0.5*(fabs(l2) + l2);
   const double gt = g2 - fri*g1;
-  C[0] = U[0] + gt*(on ? S0*is : 1.0);
+  C[0] = U[0] + gt*(none ? 1.0 : S0*is);
   C[1] = U[1] + gt*(S1*is);
   C[2] = F2 - (g1 + fri*g2);
 }
