@@ -323,9 +323,11 @@ template <typename T> struct ErrBound {
   T lo, hi;   // |dR|^2 / max(|R|^2, 1) surely at most eps^2, surely above it
   __device__ __forceinline__ explicit ErrBound(T eps)
   {
-    // the quotient and the root are within a few ulp: 1e-13 (FP64), 4e-6 (FP32)
+    // the quotient and the root are within a few ulp: 1e-13 (FP64), 4e-6 (FP32).
+    // A tolerance whose square is no normal number, and a negative one, which no
+    // change is within, leave every decision to the quotient and the root.
     const T e2 = eps*eps, m = sizeof(T) == 8 ? T(1e-13) : T(4e-6);
-    const bool ok = e2 > (sizeof(T) == 8 ? T(1e-290) : T(1e-30));
+    const bool ok = eps > T(0) && e2 > (sizeof(T) == 8 ? T(1e-290) : T(1e-30));
     lo = ok ? e2*(T(1) - m) : T(-1);
     hi = ok ? e2*(T(1) + m) : T(INFINITY);
   }
