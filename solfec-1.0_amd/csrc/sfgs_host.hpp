@@ -105,8 +105,8 @@ int reassemble(sfgs_ctx *ctx);
 // body-space operator of NEWTON_SOLVER with locdyn OFF: z = W x formed as
 // H (h M^-1 H' x) through the bodies (x at x + stride p for row p); mode 0:
 // y = beta y + alpha (X z + Y x) + alpha delta x (x 3 per row), mode 1:
-// U = B + z (U, B in SoA planes)
+// U = B + z (U, B in SoA planes); stop: as MeritArgs
 int bodyspace_product(sfgs_ctx *ctx, const double *x, int stride, int mode, const double *X, const double *Y,
-                      double alpha, double beta, double delta, double *y);
+                      double alpha, double beta, double delta, double *y, const int *stop = nullptr);
 
 } // namespace sfgs

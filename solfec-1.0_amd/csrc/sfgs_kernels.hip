@@ -1019,10 +1019,12 @@ __global__ void k_body_update(BodyView bv, ConView cv, int nb, const int *bptr, 
 
 // body-space products of NEWTON_SOLVER with locdyn OFF (U_WR_B, nts.c:396-431):
 // H_trans_R and BODY_Invvec per body, v_b = h M_b^-1 sum_c (+/-) H_c' x_c with
-// x_c at x + stride p, p = iperm[c]; obstacles carry none (bod.c:431)
+// x_c at x + stride p, p = iperm[c]; obstacles carry none (bod.c:431).  Nothing is
+// done once *stop is set (null: none).
 __global__ void k_bs_bodies(BodyView bv, ConView cv, int nb, const int *bptr, const int *blist, const int *iperm,
-                            const double *x, int stride, double step, double *v)
+                            const double *x, int stride, double step, double *v, const int *stop)
 {
+  if (stop && *stop) return;
   int b = blockIdx.x*blockDim.x + threadIdx.x;
   if (b >= nb) return;
   double f[6] = {0, 0, 0, 0, 0, 0};
@@ -1064,12 +1066,13 @@ __global__ void k_bs_bodies(BodyView bv, ConView cv, int nb, const int *bptr, co
 
 // H_times_u per row p: z = H_m v_m - H_s v_s; mode 0 the step operator of
 // Matvec (nts.c:584-652), y = beta y + alpha (X z + Y x_p) + alpha delta x_p;
-// mode 1 U = B + z
+// mode 1 U = B + z.  Nothing is done once *stop is set (null: none).
 __global__ __launch_bounds__(TPB) void k_bs_rows(BodyView bv, ConView cv, int n, const int *perm, const double *v,
                                                   int mode, const double *Xm, const double *Ym, const double *x,
                                                   double alpha, double beta, double delta, double *y,
-                                                  const double *B, double *U)
+                                                  const double *B, double *U, const int *stop)
 {
+  if (stop && *stop) return;
   int p = blockIdx.x*blockDim.x + threadIdx.x;
   if (p >= n) return;
   const int i = perm[p], m = cv.master[i], s = cv.slave[i];
@@ -1122,7 +1125,7 @@ __global__ void k_perm3(int n, const int *perm, const double *xn, double *xp)
 }
 
 int sfgs::bodyspace_product(sfgs_ctx *ctx, const double *x, int stride, int mode, const double *X, const double *Y,
-                            double alpha, double beta, double delta, double *y)
+                            double alpha, double beta, double delta, double *y, const int *stop)
 {
   const int n = ctx->nc, nb = ctx->nb;
   if (n == 0) return 0;
@@ -1134,9 +1137,9 @@ int sfgs::bodyspace_product(sfgs_ctx *ctx, const double *x, int stride, int mode
              ctx->rest.p, ctx->coh.p, ctx->Rn.p, ctx->Un.p};
   if (nb > 0)
     hipLaunchKernelGGL(k_bs_bodies, dim3(nblk(nb)), dim3(TPB), 0, st, bv, cv, nb, ctx->bptr.p, ctx->blist.p,
-                       ctx->iperm.p, x, stride, ctx->step, ctx->bsv.p);
+                       ctx->iperm.p, x, stride, ctx->step, ctx->bsv.p, stop);
   hipLaunchKernelGGL(k_bs_rows, dim3(nblk(n)), dim3(TPB), 0, st, bv, cv, n, ctx->perm.p, ctx->bsv.p, mode, X, Y, x,
-                     alpha, beta, delta, y, ctx->B.p, ctx->U.p);
+                     alpha, beta, delta, y, ctx->B.p, ctx->U.p, stop);
   HIPCHK(hipGetLastError());
   return 0;
 }
