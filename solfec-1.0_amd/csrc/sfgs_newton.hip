@@ -45,7 +45,8 @@ namespace {
   default: { constexpr int GG = 4; CALL; } break; }
 
 constexpr int NT_KDIM = 20;        // hypre_FlexGMRESCreate default k_dim (flexgmres.c:91)
-constexpr int NT_DOT_BLOCKS = 256; // partials of one dot product
+constexpr int NT_DOT_BLOCKS = 256; // most partials of one dot product
+static_assert(NT_DOT_BLOCKS <= TPB, "nt_dot_sum: one partial per thread");
 
 struct NtRows {
   int n;
@@ -64,7 +65,9 @@ struct NtRows {
 // 43 us of them on the device; now
 // 200 iterations take 9.6 ms on the device, the whole solve 12.0 ms in place of 15.4.
 struct NtCtl {
-  static const int RING = 64;
+  // RING merits are kept; the host reads them once per batch of at most BATCH iterations
+  static constexpr int RING = 64, BATCH = 32;
+  static_assert(BATCH <= RING, "a batch's merits are read before they are overwritten");
   int done, iters, nan;
   double merit;
   double hist[RING];     // merit of iteration k at k % RING
@@ -650,7 +653,7 @@ int SFGS_Newton_Solve(sfgs_ctx *ctx, const SFGS_NEWTON_PARAM *par, double *merhi
     HIPCHK(hipMemcpyAsync(ctl, &h, sizeof(h), hipMemcpyHostToDevice, st));
     const double lo = ctx->energy < DBL_EPSILON ? 1.0 : ctx->energy;
     NtTest test{ctl, 0, ctx->mpartials.p, 0, par->maxiter, lo, par->meritval};
-    for (int batch = 4; !h.done; batch = std::min(2*batch, NtCtl::RING/2))
+    for (int batch = 4; !h.done; batch = std::min(2*batch, NtCtl::BATCH))
     {
       const int last = (int)std::min((long long)test.k + batch, (long long)par->maxiter + 1);
       for (; test.k < last; test.k ++)
