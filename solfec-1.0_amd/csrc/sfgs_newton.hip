@@ -13,11 +13,15 @@
 //                theta d, R = proj(R + dr) (nts.c:1084-1093)
 //   k_nt_matvec  y = beta y + alpha (X (W x) + Y x) + alpha delta x: the
 //                operator of the linear step (Matvec, nts.c:584-652), W x
-//                over the slices with the row's lanes summed by shuffles
-//   k_nt_dot     deterministic per-block partial sums of x'y (summed on the
-//                host in block order)
-//   k_nt_axpy, k_nt_scale, k_nt_precond, k_nt_update  the vector work of
-//                flexible GMRES (ext/krylov/flexgmres.c) and R = proj(R + dr)
+//                by the gather of the sweeps (gather_rows)
+//   k_nt_dot     deterministic per-block partial sums of x'y, into host memory
+//                (the host adds them in block order)
+//   k_nt_mgs     one step of modified Gram-Schmidt, with the dot product of
+//                the next; k_nt_arnoldi the end of an Arnoldi step (norm,
+//                scaling, Givens update); k_nt_start and k_nt_cycle the start
+//                and the end of a cycle (ext/krylov/flexgmres.c)
+//   k_nt_axpy, k_nt_precond, k_nt_update  the other vector work of flexible
+//                GMRES and R = proj(R + dr)
 // The diagonal solve runs its loop on the device (NtCtl); the GMRES driver runs on the
 // host, with the Arnoldi steps and the Hessenberg system (at most 21 x 20) on the
 // device and one wait per step for the residual estimate.  All of this is HBM-bound
@@ -456,10 +460,10 @@ struct NtWork {
   }
 
   // hypre_FlexGMRESSolve (flexgmres.c:260-700) with rel_change off, cf_tol 0,
-  // r_tol 0, k_dim 20: x updated in place.  The Arnoldi step runs on the
-  // device (dot products reduced there, the Givens update in one thread); the
-  // host reads the residual estimate once per iteration and the small
-  // Hessenberg system once per cycle.
+  // r_tol 0, k_dim 20: x updated in place.  The Arnoldi steps and the solve of the
+  // Hessenberg system run on the device (dot products reduced there, the Givens
+  // update in one thread); the host reads the residual estimate once per step, the
+  // norms at a cycle's start, and the Hessenberg system only where a cycle restarts.
   // bnorm2: bb . bb
   int gmres(const double *bb, double bnorm2, double *x, int max_iter, int min_iter, double a_tol)
   {
