@@ -200,6 +200,9 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs g)
 
 static const int NF = 18, NI = 32, NH = 128, NO = 3, NOP = 32;
 
+// most K slices of a weight-gradient product (wgrad_slice)
+static const int WGRAD_SLICES = 64;
+
 struct Model {
   // FP32 master parameters, layout [in][out] per layer, then biases
   // W1 32x128, b1 128, W2 128x128, b2 128, W3 128x128, b3 128, W4 128x32, b4 32
@@ -216,7 +219,7 @@ struct Model {
   int cap = 0;
   bf16 *X = nullptr, *H1 = nullptr, *H2 = nullptr, *H3 = nullptr, *dO = nullptr, *dZ = nullptr, *dZ2 = nullptr;
   float *Z1 = nullptr, *Z2 = nullptr, *Z3 = nullptr, *O = nullptr, *Y = nullptr, *loss = nullptr;
-  float *part = nullptr;   // split-K partials of the gradient: up to wgrad_slices(cap) x total
+  float *part = nullptr;   // split-K partials of the gradient: WGRAD_SLICES x total, whatever the batch
   // device-resident training set
   float *tX = nullptr, *tY = nullptr;
   long long tn = 0, tcap = 0;
@@ -499,8 +502,9 @@ void sfgs_mlp_release(sfgs_ctx *ctx)
 // multiple of the tile's K, so that a batch of 4096 fills 128 of them (8 slices of
 // 512 left 32 workgroups with 16 dependent tile steps each: 13.0 us a product on
 // average over the pass, 8.8 with 128).  Large batches take longer slices, at most
-// 64 of them, which bounds the partials.
-static int wgrad_slice(int B) { return std::max(128, ((B + 63)/64 + BK - 1)/BK*BK); }
+// WGRAD_SLICES of them, which bounds the partials.  The count does not grow with the
+// batch: 8192 rows take 64 slices of 128, 8256 take 52 of 160.
+static int wgrad_slice(int B) { return std::max(128, ((B + WGRAD_SLICES - 1)/WGRAD_SLICES + BK - 1)/BK*BK); }
 static int wgrad_slices(int B) { return (B + wgrad_slice(B) - 1)/wgrad_slice(B); }
 
 static int gemm(sfgs_ctx *ctx, const GemmArgs &g)
@@ -534,6 +538,7 @@ static int ensure_batch(sfgs_ctx *ctx, Model *m, int B)
 {
   if (B <= m->cap) return 0;
   (void)hipStreamSynchronize(ctx->stream);
+  m->cap = 0;
   void **bufs[] = {(void**)&m->X, (void**)&m->H1, (void**)&m->H2, (void**)&m->H3, (void**)&m->dO, (void**)&m->dZ,
                    (void**)&m->dZ2, (void**)&m->Z1, (void**)&m->Z2, (void**)&m->Z3, (void**)&m->O, (void**)&m->Y,
                    (void**)&m->loss};
@@ -547,10 +552,7 @@ static int ensure_batch(sfgs_ctx *ctx, Model *m, int B)
     *bufs[k] = nullptr;
     HIPCHK(hipMalloc(bufs[k], sz[k]*(size_t)cap));
   }
-  if (m->part) (void)hipFree(m->part);
-  m->part = nullptr;
-  // a smaller batch can take more, shorter slices than the capacity: 64 at most
-  HIPCHK(hipMalloc(&m->part, sizeof(float)*m->total*64));
+  if (!m->part) HIPCHK(hipMalloc(&m->part, sizeof(float)*m->total*WGRAD_SLICES));
   m->cap = cap;
   return 0;
 }
