@@ -224,13 +224,14 @@ __device__ __forceinline__ void scf_residual(T fri, T coh, T shift, const T *U, 
 // quotients shared (1/(1 + mu^2) once, |U_T| and 1/|S_T| from one reciprocal root
 // each) instead of three roots and five divisions, which took 920 of a slice's
 // clocks.  A tangential part whose square is subnormal counts as none: u2 = (1, 0)
-// as in spectral.  What is not finite stays so, as there: 0.5 (|l| + l) carries a NaN
-// and makes one of -inf where a maximum would give 0, and a tangential part that is
-// NaN or whose square overflows is NaN and not none.  Only the merit sums depend on it.
+// as in spectral.  What is not finite stays so, as there: 0.5 (|l| + l), the half
+// taken into the shared quotient, carries a NaN and makes one of -inf where a maximum
+// would give 0, and a tangential part that is NaN or whose square overflows is NaN and
+// not none.  Only the merit sums depend on it.
 __device__ __forceinline__ void merit_residual(double fri, double coh, double shift, const double *U, const double *R,
                                                double *C)
 {
-  const double io = rcp64(1.0 + fri*fri);
+  const double ho = 0.5*rcp64(1.0 + fri*fri);
   const double uu = U[0]*U[0] + U[1]*U[1];
   const double ulen = uu < DBL_MIN ? 0.0 : uu*rsqrt64(uu);
   const double F2 = U[2] + shift + fri*ulen;
@@ -238,8 +239,8 @@ __device__ __forceinline__ void merit_residual(double fri, double coh, double sh
   const double ss = S0*S0 + S1*S1;
   const bool none = ss < DBL_MIN;
   const double is = none ? 0.0 : rsqrt64(ss), sl = ss*is;
-  const double l1 = -(S2 + fri*sl)*io, l2 = (sl - fri*S2)*io;
-  const double g1 = 0.5*(fabs(l1) + l1), g2 = 0.5*(fabs(l2) + l2);
+  const double l1 = -(S2 + fri*sl)*ho, l2 = (sl - fri*S2)*ho;   // half of each
+  const double g1 = fabs(l1) + l1, g2 = fabs(l2) + l2;
   const double gt = g2 - fri*g1;
   C[0] = U[0] + gt*(none ? 1.0 : S0*is);
   C[1] = U[1] + gt*(S1*is);
