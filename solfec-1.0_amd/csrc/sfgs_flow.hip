@@ -5,7 +5,7 @@
 // sizes of a settled packing each colour launch is a chain of dependent
 // latencies (row data, gather, 3x3 Newton) with under one wavefront per SIMD.
 // Here every wavefront owns a fixed set of slices (slice s -> wave s mod
-// nwaves) and runs them in colour-major order, sweep after sweep.  A row waits
+// nwaves; flow_waves) and runs them in colour-major order, sweep after sweep.  A row waits
 // only for its own neighbours: with ver[j] the number of sweeps row j has
 // completed, row i starts sweep k once every lower-colour neighbour j (j < i in
 // the colour-major order) has ver[j] >= k + 1 and every higher-colour
@@ -271,14 +271,26 @@ __global__ void k_flow_final(int n, const T *Rf, const T *Uf, T *R, T *U)
   for (int k = 0; k < 3; k ++) U[(size_t)k*n + p] = Uf[(size_t)k*n + p];
 }
 
+// Wavefronts of a launch over ns slices, all resident at once (3/4 of the
+// occupancy's count), but no more than one per CU for every 10 slices per CU, and
+// at most three.  Every wavefront adds to the counter and the partials of each
+// sweep's test and polls its neighbours' versions meanwhile, so more of them than
+// the slices need make a sweep longer, not shorter.  us a sweep in FP64 with two
+// lanes a row (256 CUs) for 256, 512, 768 and 1536 wavefronts: 12k rows 47, 51, 86,
+// 86; 41k rows 60, 65, 82, 144; 96k rows 90, 77, 88, 140; 188k rows 154, 106, 103,
+// 146; 432k rows 472, 289, 240, 250.
+constexpr int FLOW_SLICES = 10, FLOW_PER_CU = 3;
+
 template <typename T>
-static int flow_cap(sfgs_ctx *ctx, int G, int *cap)
+static int flow_waves(sfgs_ctx *ctx, int G, int ns, int *nwaves)
 {
   int nb = 0, cus = 0;
   const void *kern = G == 2 ? (const void*)k_flow<T, 2> : (const void*)k_flow<T, 1>;
   HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern, 64, 0));
   HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
-  *cap = (nb * cus * 3) / 4;   // every wavefront must be resident at once
+  const int resident = (nb * cus * 3) / 4;   // every wavefront must be resident at once
+  const int percu = std::min((ns + FLOW_SLICES*cus - 1) / (FLOW_SLICES*cus), FLOW_PER_CU);
+  *nwaves = std::max(1, std::min({resident, percu*cus, ns}));
   return 0;
 }
 
@@ -291,9 +303,8 @@ static int run_flow_t(sfgs_ctx *ctx, const SweepArgs<T> &sa, T *X0, T *X1, int m
   std::memset(&hc, 0, sizeof(hc));
   if (G != 1 && G != 2) { ctx->err = "the flow schedule supports 1 or 2 lanes per row"; return SFGS_E_STATE; }
   if (n == 0 || ns == 0) { hc.done = 1; return 0; }
-  int cap = 0;
-  CHK(flow_cap<T>(ctx, G, &cap));
-  const int nwaves = std::max(1, std::min(cap, ns));
+  int nwaves = 0;
+  CHK(flow_waves<T>(ctx, G, ns, &nwaves));
   // device scratch: third R buffer, U and merit-U pairs, row versions, partials, counters
   const size_t bR = sizeof(T)*4*(size_t)n, bU = sizeof(T)*3*(size_t)n;
   const size_t off_ver = bR + 4*bU, off_part = off_ver + sizeof(int)*(size_t)n + 64;
