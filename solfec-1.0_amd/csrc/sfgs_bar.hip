@@ -210,7 +210,11 @@ static int bar_cap(sfgs_ctx *ctx, int G, int *cap)
   const void *kern = G == 2 ? (const void*)k_bar<T, 2> : (const void*)k_bar<T, 1>;
   HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern, BAR_NW*64, 0));
   HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
-  *cap = (nb * cus * 3) / 4;   // every workgroup must be resident at once
+  // Every workgroup must be resident at once.  One per CU at most, whatever fits: each
+  // barrier waits for all of them.  us a sweep at 432k rows for 192 and 384 workgroups:
+  // one lane a row 356 and 451 (FP64), 231 and 323 (FP32), two lanes 225 and 329 (FP32;
+  // two do not fit in FP64); the same below 100k rows.
+  *cap = (std::min(nb, 1) * cus * 3) / 4;
   return 0;
 }
 
