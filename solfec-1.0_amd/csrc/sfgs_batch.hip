@@ -676,6 +676,9 @@ static int batch_solve(sfgs_ctx *ctx, const SFGS_PARAM *par, const SFGS_BATCH_TU
   hipStream_t st = ctx->stream;
   const int nsc = ctx->nscenes, ncol = ctx->ncolours, n = ctx->nc;
   const bool mixed = par->precision == SFGS_PREC_MIXED;
+  // the per-colour schedule, which every MIXED solve takes (its FP64 phase runs per
+  // scene), or launches over chunks of scenes that fit the resident capacity
+  const bool per_colour = tn.schedule == 1 || mixed;
   const int G = tn.lanes_per_row, NW = tn.waves_per_group;
   const int ng = nsc*ncol;
   if ((int)ctx->h_colptr.size() != ng + 1 || (int)ctx->h_cslice.size() != ng + 1)
@@ -683,6 +686,7 @@ static int batch_solve(sfgs_ctx *ctx, const SFGS_PARAM *par, const SFGS_BATCH_TU
     ctx->err = "layout tables do not match the scenes";
     return SFGS_E_STATE;
   }
+  CHK(set_halves(ctx, per_colour));
 
   // workgroups per scene (the persistent launch runs FP64 solves only)
   int cap = 0;
@@ -756,10 +760,7 @@ static int batch_solve(sfgs_ctx *ctx, const SFGS_PARAM *par, const SFGS_BATCH_TU
     bf.X0 = ctx->R32.p; bf.X1 = ctx->R32b.p; bf.Ut = ctx->U32.p; bf.Umt = ctx->Um32.p;
   }
 
-  // launches over chunks of scenes that fit the resident capacity, or the per-colour
-  // schedule, which every MIXED solve takes (its FP64 phase runs per scene)
   std::vector<int> wgs((size_t)nsc, 0);
-  const bool per_colour = tn.schedule == 1 || mixed;
   HIPCHK(hipEventRecord(ctx->ev0, st));
   if (per_colour)
   {

@@ -87,6 +87,7 @@ struct sfgs_ctx {
   sfgs::DBuf<long long> slice_off;       // block offset of slice (in blocks, multiple of 64)
   sfgs::DBuf<long long> slice_lens;      // build_order: block slots of every slice, for the offsets
   sfgs::DBuf<sfgs::SliceTab> slice_tab;  // the four together, for the sweeps
+  bool halves = true;                    // smaller colours in slices of half the rows (sfgs::set_halves)
   long long sell_blocks = 0;             // total block slots, the last slot of each slice filled up
 
   // ---- permuted row data (colour-major order)

@@ -98,6 +98,9 @@ int run_bar(sfgs_ctx *ctx, const SweepArgs<double> &sa, double *X0, double *X1, 
 int run_bar(sfgs_ctx *ctx, const SweepArgs<float> &sa, float *X0, float *X1, int maxiter, int nomerit,
             double eps, double meritval, int reverse, double *hist, Ctrl &hc, float *ms);
 
+// slices of half the rows in the smaller colours, or 64/G rows in all (sfgs_kernels.hip):
+// what the next solve's schedule takes; the blocks move, rows, R and U stay where they are
+int set_halves(sfgs_ctx *ctx, bool halves);
 // FP32 copies of the sweep data (sfgs_kernels.hip)
 int build_f32_mirror(sfgs_ctx *ctx);
 // re-run the assembly of the current bodies and contacts (after a layout change)

@@ -493,6 +493,15 @@ __global__ __launch_bounds__(TPB) void k_slice_len(int ns, const int *row0, cons
   if (l == 63) { slen[s] = sum; slen_ll[s] = (long long)((sum + SLICE - 1) / SLICE) * SLICE; }
 }
 
+// per slice (one wavefront): the block slot of each row's first block
+__global__ __launch_bounds__(TPB) void k_row_slot(int ns, const SliceTab *tab, const int *rowoff, long long *slot)
+{
+  const int s = blockIdx.x*(TPB/SLICE) + (threadIdx.x >> 6), l = threadIdx.x & 63;
+  if (s >= ns || l >= tab[s].nrows) return;
+  const int p = tab[s].row0 + l;
+  slot[p] = tab[s].off + rowoff[p];
+}
+
 __global__ void k_slice_tab(int ns, const int *row0, const int *nrows, const int *slen, const long long *off, SliceTab *tab)
 {
   const int s = blockIdx.x*blockDim.x + threadIdx.x;
@@ -615,6 +624,27 @@ __device__ __forceinline__ int slice_row_of(int rowoff, int nr, int q)
     if (m < nr && v <= q) lo = m;
   }
   return lo;
+}
+
+// the blocks of a layout into slices of other rows (the same rows in the same
+// order): slot holds the place of each row's first block in W0 and wcol0
+__global__ __launch_bounds__(TPB) void k_repack(int ns, SellOut so, const long long *slot, const double *W0, const int *wcol0)
+{
+  const int s = blockIdx.x*(TPB/SLICE) + (threadIdx.x >> 6), l = threadIdx.x & 63;
+  if (s >= ns) return;
+  const int row0 = so.row0[s], nr = so.nrows[s], total = so.slen[s], ro = l < nr ? so.rowoff[row0 + l] : 0;
+  const long long off = so.off[s];
+  for (int q0 = 0; q0 < total; q0 += SLICE)
+  {
+    const int k = q0 + l, r = slice_row_of(ro, nr, k), first = __shfl(ro, r, 64);
+    const bool on = k < total;
+    const long long q = on ? slot[row0 + r] + (k - first) : 0;
+    const double *src = W0 + 9*(q & ~63LL) + (q & 63);
+    double *Wb = so.W + 9*(off + q0) + l;
+#pragma unroll
+    for (int e = 0; e < 9; e ++) Wb[e*SLICE] = on ? src[e*SLICE] : 0.0;
+    so.wcol[off + k] = on ? wcol0[q] : 0;
+  }
 }
 
 // off-diagonal blocks W_ij = h s_i s_j H_i^b iM_b H_j^b' (ldy.c:738-844).  One
@@ -1396,11 +1426,69 @@ static int colour_graph(sfgs_ctx *ctx, int n, bool symmetric)
 // 76.2 and 76.4: more partial sums to add up at the end), and so do halves in the
 // group launch (216 rows 46.3 and 51.6).  1024 in place of 512: 200k 203.4, 60001
 // 103.3.  The iterates do not depend on it.
+// Not for the persistent batch launch (halves = false), where a few wavefronts take all
+// slices of a scene in turn: 24 scenes of 27 to 1000 spheres in 60 sweeps with two lanes
+// a row, one workgroup per 1024 rows, halves and full slices: 15.5 and 9.0 ms with one
+// wavefront in it, 9.4 and 6.0 with two, 6.2 and 4.7 with four, 5.1 and 4.2 with eight;
+// by colours 6.6 and 6.9 ms (100 sweeps).
 static const int GROUP_NW = 4, HALF_SLICES = 512;
-static int slice_rows(int n, int G)
+static int slice_rows(int n, int G, bool halves)
 {
   const int full = SLICE / G, half = full / 2;
-  return n > GROUP_NW*full && n <= HALF_SLICES*half ? half : full;
+  return halves && n > GROUP_NW*full && n <= HALF_SLICES*half ? half : full;
+}
+
+// rows per slice of every colour of the rows in ctx->h_colptr
+static std::vector<int> slice_plan(const sfgs_ctx *ctx, bool halves)
+{
+  const int ncol = ctx->ncolours, nc = (int)ctx->h_colptr.size() - 1;
+  std::vector<int> rps((size_t)std::max(ncol, 1), 0);
+  for (int c = 0; c < nc; c ++) rps[c % ncol] += ctx->h_colptr[c + 1] - ctx->h_colptr[c];
+  for (int &r : rps) r = slice_rows(r, ctx->G_built, halves);
+  return rps;
+}
+
+// the slices of the ordered rows, and room for their blocks
+static int build_slices(sfgs_ctx *ctx)
+{
+  const int ncol = ctx->ncolours, nc = (int)ctx->h_colptr.size() - 1;
+  const std::vector<int> rps = slice_plan(ctx, ctx->halves);
+  std::vector<int> row0, nrows;
+  ctx->h_cslice.assign((size_t)nc + 1, 0);
+  for (int c = 0; c < nc; c ++)
+  {
+    const int m = rps[c % ncol];
+    for (int r = ctx->h_colptr[c]; r < ctx->h_colptr[c + 1]; r += m)
+    {
+      row0.push_back(r);
+      nrows.push_back(std::min(m, ctx->h_colptr[c + 1] - r));
+    }
+    ctx->h_cslice[c + 1] = (int)row0.size();
+  }
+  int ns = (int)row0.size();
+  ctx->nslices = ns;
+  CHK(upload(ctx, ctx->slice_row0, row0.data(), (size_t)ns));
+  CHK(upload(ctx, ctx->slice_nrows, nrows.data(), (size_t)ns));
+  CHK(ensure(ctx, ctx->slice_len, (size_t)ns + 1));
+  CHK(ensure(ctx, ctx->slice_off, (size_t)ns + 1));
+  DBuf<long long> &lens = ctx->slice_lens;
+  CHK(ensure(ctx, lens, (size_t)ns + 1));
+  HIPCHK(hipMemsetAsync(lens.p, 0, sizeof(long long)*((size_t)ns + 1), ctx->stream));
+  if (ns > 0)
+    hipLaunchKernelGGL(k_slice_len, dim3(nblk((long long)ns*SLICE)), dim3(TPB), 0, ctx->stream, ns, ctx->slice_row0.p,
+                       ctx->slice_nrows.p, ctx->perm.p, ctx->rowptr.p, ctx->rowoff.p, ctx->slice_len.p, lens.p);
+  CHK(scan_ll(ctx, lens.p, ctx->slice_off.p, ns + 1));
+  CHK(ensure(ctx, ctx->slice_tab, (size_t)ns));
+  if (ns > 0)
+    hipLaunchKernelGGL(k_slice_tab, dim3(nblk(ns)), dim3(TPB), 0, ctx->stream, ns, ctx->slice_row0.p, ctx->slice_nrows.p,
+                       ctx->slice_len.p, ctx->slice_off.p, ctx->slice_tab.p);
+  long long total = 0;
+  HIPCHK(hipMemcpyAsync(&total, ctx->slice_off.p + ns, sizeof(long long), hipMemcpyDeviceToHost, ctx->stream));
+  HIPCHK(hipStreamSynchronize(ctx->stream));
+  ctx->sell_blocks = total;
+  CHK(ensure(ctx, ctx->W, (size_t)(9*total)));
+  CHK(ensure(ctx, ctx->wcol, (size_t)total));
+  return 0;
 }
 
 // permutation into colour-major order and the slice table
@@ -1464,45 +1552,8 @@ static int build_order(sfgs_ctx *ctx, int n, bool have_master)
   if (nc > 0) HIPCHK(hipMemcpyAsync(cnt.data(), ctx->counter.p, sizeof(int)*(size_t)nc, hipMemcpyDeviceToHost, ctx->stream));
   HIPCHK(hipStreamSynchronize(ctx->stream));
   ctx->h_colptr.assign((size_t)nc + 1, 0);
-  ctx->h_cslice.assign((size_t)nc + 1, 0);
-  std::vector<int> row0, nrows, rps((size_t)std::max(ncol, 1), 0);
-  for (int c = 0; c < nc; c ++) rps[c % ncol] += cnt[c];
-  for (int &r : rps) r = slice_rows(r, G);
-  for (int c = 0; c < nc; c ++)
-  {
-    ctx->h_colptr[c + 1] = ctx->h_colptr[c] + cnt[c];
-    const int m = rps[c % ncol];
-    for (int r = ctx->h_colptr[c]; r < ctx->h_colptr[c + 1]; r += m)
-    {
-      row0.push_back(r);
-      nrows.push_back(std::min(m, ctx->h_colptr[c + 1] - r));
-    }
-    ctx->h_cslice[c + 1] = (int)row0.size();
-  }
-  int ns = (int)row0.size();
-  ctx->nslices = ns;
-  CHK(upload(ctx, ctx->slice_row0, row0.data(), (size_t)ns));
-  CHK(upload(ctx, ctx->slice_nrows, nrows.data(), (size_t)ns));
-  CHK(ensure(ctx, ctx->slice_len, (size_t)ns + 1));
-  CHK(ensure(ctx, ctx->slice_off, (size_t)ns + 1));
-  DBuf<long long> &lens = ctx->slice_lens;
-  CHK(ensure(ctx, lens, (size_t)ns + 1));
-  HIPCHK(hipMemsetAsync(lens.p, 0, sizeof(long long)*((size_t)ns + 1), ctx->stream));
-  if (ns > 0)
-    hipLaunchKernelGGL(k_slice_len, dim3(nblk((long long)ns*SLICE)), dim3(TPB), 0, ctx->stream, ns, ctx->slice_row0.p,
-                       ctx->slice_nrows.p, ctx->perm.p, ctx->rowptr.p, ctx->rowoff.p, ctx->slice_len.p, lens.p);
-  CHK(scan_ll(ctx, lens.p, ctx->slice_off.p, ns + 1));
-  CHK(ensure(ctx, ctx->slice_tab, (size_t)ns));
-  if (ns > 0)
-    hipLaunchKernelGGL(k_slice_tab, dim3(nblk(ns)), dim3(TPB), 0, ctx->stream, ns, ctx->slice_row0.p, ctx->slice_nrows.p,
-                       ctx->slice_len.p, ctx->slice_off.p, ctx->slice_tab.p);
-  long long total = 0;
-  HIPCHK(hipMemcpyAsync(&total, ctx->slice_off.p + ns, sizeof(long long), hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(hipStreamSynchronize(ctx->stream));
-  ctx->sell_blocks = total;
-  CHK(ensure(ctx, ctx->W, (size_t)(9*total)));
-  CHK(ensure(ctx, ctx->wcol, (size_t)total));
-  return 0;
+  for (int c = 0; c < nc; c ++) ctx->h_colptr[c + 1] = ctx->h_colptr[c] + cnt[c];
+  return build_slices(ctx);
 }
 
 static int ensure_rows(sfgs_ctx *ctx, int n)
@@ -2077,6 +2128,45 @@ static int run_gs(sfgs_ctx *ctx, SweepArgs<T> sa, T *X0, T *X1, int maxiter, int
 }
 
 // FP32 copies of the sweep data (built once per assembled system)
+int sfgs::set_halves(sfgs_ctx *ctx, bool halves)
+{
+  if (ctx->halves == halves) return 0;
+  const int n = ctx->nc;
+  if (n == 0 || slice_plan(ctx, halves) == slice_plan(ctx, ctx->halves)) { ctx->halves = halves; return 0; }
+  // slices of half the rows fill at most one more slot each; without the room for a
+  // second copy of the blocks the layout stays as it is (it holds for any schedule)
+  const size_t slots = (size_t)ctx->sell_blocks + (size_t)SLICE*(size_t)(2*ctx->nslices);
+  DBuf<double> W;
+  DBuf<int> wcol;
+  DBuf<long long> slot;
+  const std::string err = ctx->err;
+  if (ensure(ctx, W, 9*slots) || ensure(ctx, wcol, slots) || ensure(ctx, slot, (size_t)n))
+  {
+    (void)hipGetLastError();
+    ctx->err = err;
+    release(W); release(wcol); release(slot);
+    return 0;
+  }
+  hipLaunchKernelGGL(k_row_slot, dim3(nblk((long long)ctx->nslices*SLICE)), dim3(TPB), 0, ctx->stream, ctx->nslices,
+                     ctx->slice_tab.p, ctx->rowoff.p, slot.p);
+  std::swap(W, ctx->W);
+  std::swap(wcol, ctx->wcol);
+  ctx->halves = halves;
+  ctx->mirror_valid = 0;
+  ctx->assembled = 0;   // until the blocks are in their new places
+  int rc = build_slices(ctx);
+  if (!rc)
+    hipLaunchKernelGGL(k_repack, dim3(nblk((long long)ctx->nslices*SLICE)), dim3(TPB), 0, ctx->stream, ctx->nslices,
+                       sell_out(ctx), slot.p, W.p, wcol.p);
+  const hipError_t e = hipStreamSynchronize(ctx->stream);
+  release(W); release(wcol); release(slot);
+  if (rc) return rc;
+  HIPCHK(e);
+  HIPCHK(hipGetLastError());
+  ctx->assembled = 1;
+  return 0;
+}
+
 int sfgs::build_f32_mirror(sfgs_ctx *ctx)
 {
   if (ctx->mirror_valid) return 0;
@@ -2140,6 +2230,7 @@ int SFGS_Solve(sfgs_ctx *ctx, const SFGS_PARAM *par, double *rerhist, double *me
   if (ctx->upmin) { ctx->err = "the local dynamics hold the diagonal blocks only (SFGS_Locdyn_Update_Min)"; return SFGS_E_STATE; }
   if (ctx->nscenes > 1) { ctx->err = "the system holds independent scenes: use SFGS_Batch_Solve"; return SFGS_E_STATE; }
   HIPCHK(hipSetDevice(ctx->device));
+  CHK(sfgs::set_halves(ctx, true));
   hipStream_t st = ctx->stream;
   const int ncol = ctx->ncolours, maxiter = par->maxiter, n = ctx->nc;
   const int nomerit = par->meritval >= 1.0 ? 1 : 0;
