@@ -763,9 +763,9 @@ __device__ void finish_sweep(Ctrl *ctrl, const double *partials, int np, double 
 // The slice table, the stop flag, the slices and nb come first: they are in registers
 // when a wavefront starts (the preloaded arguments of the Makefile), so that its table
 // entry is on the way while the other arguments are fetched; both are misses of 0.6 us in
-// a launch of 6 to 8.  us a sweep without and with: 1000 rows 71.9 and 70.6, 7919 rows
-// 88.0 and 85.3, 60001 ellipsoids 100.2 and 98.2, 200k 192.3 and 186.5, mixed 107.6 and
-// 105.7.
+// a launch of 6 to 8.  us a sweep without and with: 2.0k rows 71.9 and 70.6, 16k rows
+// 88.0 and 85.3, 125k rows of ellipsoids 100.2 and 98.2, 417k rows 192.3 and 186.5, the
+// same in FP32 107.6 and 105.7.
 // nb: the launch's workgroups (an argument: gridDim would be a load of its own).
 // fin (the last launch of a sweep only): the block that completes the launch
 // last takes the sweep's termination test, as k_finish would after it
@@ -1417,14 +1417,14 @@ static int colour_graph(sfgs_ctx *ctx, int n, bool symmetric)
 // One CU's misses are what bounds that launch (the gather of a slice takes 3-4k
 // cycles alone and 18-21k beside six others there), so only colours with one slice
 // per SIMD of the CU are worth the launch they save; 8, 4, 3, 2 slices measured in
-// us a sweep: 216 rows 44.9, 43.9, 47.0, 51.4; 1000 rows 74.4, 71.9, 72.4, 73.2; 7919
-// rows 93.4, 88.0, 87.7, 87.6; 200k 200.6, 193.4, 192.5, 193.3.
-// Halves, in us a sweep (with a group of 8), 64/G rows against this: 7919 rows 100.0 and
-// 93.2, 60001 ellipsoids 104.4 and 101.9, 200k 206.4 and 201.6, 200k mixed 111.2
-// and 108.5; 1000 and 1331 rows the same.  Quarters or eighths add nothing there
-// and cost where colours are small (1331 rows 61.8, 63.8 and 69.7; 1000 rows 74.4,
+// us a sweep: 425 rows 44.9, 43.9, 47.0, 51.4; 2.0k rows 74.4, 71.9, 72.4, 73.2; 16k
+// rows 93.4, 88.0, 87.7, 87.6; 417k rows 200.6, 193.4, 192.5, 193.3.
+// Halves, in us a sweep (with a group of 8), 64/G rows against this: 16k rows 100.0 and
+// 93.2, 125k rows of ellipsoids 104.4 and 101.9, 417k rows 206.4 and 201.6, the same in
+// FP32 111.2 and 108.5; 2.0k and 2.7k rows the same.  Quarters or eighths add nothing
+// there and cost where colours are small (2.7k rows 61.8, 63.8 and 69.7; 2.0k rows 74.4,
 // 76.2 and 76.4: more partial sums to add up at the end), and so do halves in the
-// group launch (216 rows 46.3 and 51.6).  1024 in place of 512: 200k 203.4, 60001
+// group launch (425 rows 46.3 and 51.6).  1024 in place of 512: 417k rows 203.4, 125k
 // 103.3.  The iterates do not depend on it.
 // Not for the persistent batch launch (halves = false), where a few wavefronts take all
 // slices of a scene in turn: 24 scenes of 27 to 1000 spheres in 60 sweeps with two lanes

@@ -65,7 +65,7 @@ struct NtRows {
 
 // The control block of a diagonal Newton solve, whose loop is tested on the device:
 // the host enqueues iterations ahead and reads this once per batch of them.  With a
-// read-back of the merit's partial sums an iteration each took 70 us at 64000 rows,
+// read-back of the merit's partial sums an iteration each took 70 us at 133k rows,
 // 43 us of them on the device; now
 // 200 iterations take 9.6 ms on the device, the whole solve 12.0 ms in place of 15.4.
 struct NtCtl {
@@ -280,10 +280,10 @@ __device__ __forceinline__ double nt_dot_sum(const double *part, int np)
 // One modified Gram-Schmidt step: y -= h x0 with h the dot product whose partial
 // sums the launch before left in p0 (kept in *out; x0 null: no update), then the
 // partial sums of x1 . y (x1 null: of y . y) into p1.  A step is bound by its
-// launches (3 us each for 60k values), so the update, the sum of the partials and the
+// launches (3-4 us each for 124k values), so the update, the sum of the partials and the
 // next product are one launch instead of three, the step's end one
-// instead of five, and what the host needs is written to its memory: 11 linearisations of
-// 20011 contacts in body space with 62 steps took 10.6 ms and take 6.8.
+// instead of five, and what the host needs is written to its memory: 12 linearisations of
+// 41k contacts in body space with 62 steps took 10.6 ms and take 6.8.
 __global__ __launch_bounds__(TPB) void k_nt_mgs(long long N, const double *x0, const double *p0, double *out,
                                                  const double *x1, double *y, double *p1)
 {
